@@ -33,6 +33,13 @@ struct StepArgs {
   // [kStatusNonFinite] set to 1 when a macro-writing pass meets a non-finite
   // density or velocity; [kStatusOverflow] when a cell-list bin was full
   uint32_t* status;
+  void* f2;  // the spare population buffer of multi-step launches, or null
+  int32_t main;  // a flag with BGK or BGKGuo and nothing else (the fluid), or 0
+  // flags as bits: bounce-back without collision; any other boundary; main's
+  // collision; another collision
+  struct Classes {
+    uint32_t bounce, face, same, other;
+  } cls;
 };
 
 constexpr int kStatusNonFinite = 0;
@@ -50,6 +57,25 @@ struct LaunchShape {
 
 hipError_t launch_aa_step(int lattice, int storage, bool odd, const StepArgs& a,
                           const LaunchShape& shape, hipStream_t s);
+
+// ---- several steps per launch (multi_step.hip) ---------------------------------
+// `steps` D2Q9 steps on tiles of tx x ty cells, from one population buffer to
+// another, both in the natural layout (phase 0).  The operators are boundaries
+// with BGK, BGKGuo or no collision, and no macros are written.
+struct MultiShape {
+  int32_t id, steps, tx, ty;
+};
+// the shapes for a launch over `cells` cells, longest first
+struct MultiPlan {
+  int32_t n;
+  MultiShape shape[3];
+};
+MultiPlan multi_plan(int storage, uint64_t cells);
+hipError_t launch_multi(int storage, const MultiShape& sh, const StepArgs& a, const void* from, void* to,
+                        hipStream_t s);
+struct BatchArgs;
+// b.tiles: member and tile coordinates x | y << 16; flip: from the spare buffers back
+hipError_t launch_multi_batch(int storage, const MultiShape& sh, const BatchArgs& b, int flip, hipStream_t s);
 
 // *p = v and *p += v, in stream order (a step index that captured launches read)
 hipError_t launch_set_u64(uint64_t* p, uint64_t v, hipStream_t s);

@@ -148,7 +148,13 @@ struct lbm_ctx {
   void* u_prev = nullptr;
   double* res_partial = nullptr;
   double* res_out = nullptr;
+  // multi-step launches (D2Q9): the buffer they write to before they come back
+  // to f, asked for once; one_step while a launch shape was set by hand
+  void* f2 = nullptr;
+  bool f2_asked = false;
+  bool one_step = false;
   size_t tsz() const { return compute_double(storage) ? 8 : 4; }
+  size_t fbytes() const { return size_t(Q) * Np * storage_bytes(storage); }
 };
 
 namespace {
@@ -351,6 +357,30 @@ lbm_status particle_pass(lbm_ctx* c, uint64_t t) {
   return LBM_OK;
 }
 
+// StepArgs::main, the first flag that collides by BGK or BGKGuo and does
+// nothing else (a driver's fluid), and the flags by what they do.
+void classify(const lbm_ctx* c, StepArgs& a) {
+  for (int k = 1; k < kMaxOps && !a.main; ++k) {
+    const OpDev& o = c->ops_h[k];
+    if (c->has_op[k] && o.bc == LBM_BC_NONE &&
+        (o.coll == LBM_COLL_BGK || (o.coll == LBM_COLL_BGK_GUO && !(o.flags & LBM_OPF_GUO_CELL_FORCE))))
+      a.main = k;
+  }
+  const OpDev& m = c->ops_h[a.main];
+  for (int k = 1; k < kMaxOps; ++k) {
+    const OpDev& o = c->ops_h[k];
+    if (!c->has_op[k]) continue;
+    const uint32_t bit = 1u << k;
+    if (o.bc == LBM_BC_BOUNCE_BACK && o.coll == LBM_COLL_NONE) a.cls.bounce |= bit;
+    else if (o.bc != LBM_BC_NONE) a.cls.face |= bit;
+    if (o.coll == LBM_COLL_NONE) continue;
+    bool same = a.main && o.coll == m.coll && o.omega == m.omega;
+    if (o.coll == LBM_COLL_BGK_GUO)
+      same = same && !(o.flags & LBM_OPF_GUO_CELL_FORCE) && std::memcmp(o.vec, m.vec, sizeof o.vec) == 0;
+    (same ? a.cls.same : a.cls.other) |= bit;
+  }
+}
+
 // t_dev: where captured launches find the step index of the first step they
 // replay (t is then the offset from it), else null
 StepArgs step_args(const lbm_ctx* c, uint64_t t, bool write_macros, const uint64_t* t_dev = nullptr) {
@@ -376,7 +406,62 @@ StepArgs step_args(const lbm_ctx* c, uint64_t t, bool write_macros, const uint64
   a.t_dev = t_dev;
   a.write_macros = write_macros ? 1 : 0;
   a.status = c->status_d;
+  a.f2 = c->f2;
+  classify(c, a);
   return a;
+}
+
+// Whether whole groups of steps may run in one launch (launch_multi): a D2Q9
+// lattice whose operators read and write nothing but its populations.
+bool multi_operators(const lbm_ctx* c) {
+  if (c->lattice != LBM_D2Q9) return false;
+  for (int k = 0; k < kMaxOps; ++k)
+    if (c->has_op[k] && c->ops_h[k].coll != LBM_COLL_NONE && c->ops_h[k].coll != LBM_COLL_BGK &&
+        c->ops_h[k].coll != LBM_COLL_BGK_GUO)
+      return false;
+  return true;
+}
+
+// A spare buffer of `bytes`, or null where it would leave less than a quarter
+// of the GPU's memory free: the one-step kernels need none.
+void* spare_buffer(size_t bytes) {
+  size_t free_b = 0, total = 0;
+  void* p = nullptr;
+  if (hipMemGetInfo(&free_b, &total) != hipSuccess || free_b < bytes || free_b - bytes < total / 4 ||
+      hipMalloc(&p, bytes) != hipSuccess) {
+    (void)hipGetLastError();
+    return nullptr;
+  }
+  return p;
+}
+
+// The shapes of this lattice's multi-step launches (n = 0: it has none).
+MultiPlan multi_of(lbm_ctx* c) {
+  MultiPlan plan;
+  std::memset(&plan, 0, sizeof plan);
+  if (c->one_step || c->np > 0 || !multi_operators(c)) return plan;
+  if (!c->f2_asked) {
+    c->f2_asked = true;
+    c->f2 = spare_buffer(c->fbytes());
+  }
+  if (c->f2 && c->n[1] < 65536) plan = multi_plan(c->storage, c->N);
+  return plan;
+}
+
+// The longest pair of launches of the plan within `steps` steps, or null.
+const MultiShape* multi_fit(const MultiPlan& plan, uint64_t steps) {
+  for (int i = 0; i < plan.n; ++i)
+    if (2u * uint64_t(plan.shape[i].steps) <= steps) return &plan.shape[i];
+  return nullptr;
+}
+
+// 2 * sh.steps steps from phase 0: into the spare buffer and back
+lbm_status multi_pass(lbm_ctx* c, const MultiShape& sh, uint64_t t, const uint64_t* t_dev = nullptr) {
+  StepArgs a = step_args(c, t, false, t_dev);
+  HIP_TRY(launch_multi(c->storage, sh, a, c->f, c->f2, c->stream));
+  a.t = t + uint64_t(sh.steps);
+  HIP_TRY(launch_multi(c->storage, sh, a, c->f2, c->f, c->stream));
+  return LBM_OK;
 }
 
 // u_into: where this pass writes the velocity when it writes macros (null:
@@ -418,12 +503,13 @@ void append_bytes(std::vector<uint8_t>& k, const X& x) {
 // *t_dev by its length, so one graph serves every start step, inside the
 // ramps or past them; *t_dev is set only where a replay does not continue
 // the previous one.
-lbm_status replay_steps(lbm_ctx* c, uint64_t t, bool every) {
+lbm_status replay_steps(lbm_ctx* c, uint64_t t, bool every, const MultiPlan& multi) {
   if (!c->t_dev) HIP_TRY(hipMalloc((void**)&c->t_dev, sizeof(uint64_t)));
   std::vector<uint8_t> key;
   append_bytes(key, step_args(c, 0, every, c->t_dev));
   append_bytes(key, c->shape);
   append_bytes(key, c->steps_per_graph);
+  append_bytes(key, multi);
   append_bytes(key, c->np);
   if (c->np > 0) {
     ParticleArgs pa = particle_args(c);
@@ -439,9 +525,16 @@ lbm_status replay_steps(lbm_ctx* c, uint64_t t, bool every) {
     hipGraph_t g = nullptr;
     HIP_TRY(hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
     lbm_status s = LBM_OK;
-    for (uint32_t i = 0; i < c->steps_per_graph && !s; ++i) {
+    for (uint32_t i = 0; i < c->steps_per_graph && !s;) {
+      const MultiShape* sh = c->phase == 0 ? multi_fit(multi, c->steps_per_graph - i) : nullptr;
+      if (sh) {
+        s = multi_pass(c, *sh, i, c->t_dev);
+        i += 2u * uint32_t(sh->steps);
+        continue;
+      }
       if (c->np > 0) s = particle_pass(c, i);
       if (!s) s = fluid_pass(c, i, every, c->t_dev);
+      ++i;
     }
     if (!s && launch_add_u64(c->t_dev, c->steps_per_graph, c->stream) != hipSuccess)
       s = fail(LBM_ERR_CRITICAL, "step index advance");
@@ -548,7 +641,7 @@ lbm_status lbm_ctx_destroy(lbm_ctx* c) {
   if (c->stream) (void)hipStreamSynchronize(c->stream);
   void* ptrs[] = {c->f, c->flags, c->ops, c->rho, c->u, c->force, c->por, c->bcvel, c->pn, c->pd,
                   c->parts, c->snap, c->f64, c->t64, c->partial, c->cl_count, c->cl_slot,
-                  c->cl_overflow, c->owner, c->t_dev, c->u_prev, c->res_partial, c->res_out, c->boxes};
+                  c->cl_overflow, c->owner, c->t_dev, c->u_prev, c->res_partial, c->res_out, c->boxes, c->f2};
   for (void* p : ptrs)
     if (p) (void)hipFree(p);
   if (c->status_h) (void)hipHostFree(c->status_h);
@@ -862,6 +955,7 @@ lbm_status lbm_step(lbm_ctx* c, uint64_t t0, uint64_t nsteps) {
   s = report_faults(c);  // of earlier calls' work that has run
   if (s) return s;
   HIP_TRY(hipSetDevice(c->device));
+  const MultiPlan multi = multi_of(c);
   HIP_TRY(hipEventRecord(c->ev0, c->stream));
   s = prepare_sweep(c);  // (outside any step graph)
   if (s) return s;
@@ -879,9 +973,17 @@ lbm_status lbm_step(lbm_ctx* c, uint64_t t0, uint64_t nsteps) {
     // a whole graph of steps: from phase 0, and never the last step of the
     // call (it writes the macros), nor the one before it when tracking
     if (G > 0 && c->phase == 0 && nsteps - k > G + (track ? 1u : 0u)) {
-      s = replay_steps(c, t, every);
+      s = replay_steps(c, t, every, multi);
       if (s) return s;
       k += G;
+      continue;
+    }
+    const uint64_t silent = nsteps - k - 1;  // steps before the one that writes the macros
+    const MultiShape* sh = c->phase == 0 ? multi_fit(multi, track && silent > 0 ? silent - 1 : silent) : nullptr;
+    if (sh) {
+      s = multi_pass(c, *sh, t);
+      if (s) return s;
+      k += 2u * uint64_t(sh->steps);
       continue;
     }
     if (c->np > 0) {
@@ -983,6 +1085,7 @@ lbm_status lbm_set_step_tuning(lbm_ctx* c, const lbm_step_tuning* t) {
   c->shape.by = 1;
   c->shape.form[0] = t->form[0];
   c->shape.form[1] = t->form[1];
+  c->one_step = true;  // every step in this shape
   return LBM_OK;
 }
 
@@ -1385,6 +1488,16 @@ struct lbm_batch {
   size_t tiles_cap = 0;
   bool tiles_dirty = true;
   // captured chains: key = (length, with residual)
+  // multi-step launches: their work list (active members' tiles) and one spare
+  // buffer for every member's populations; one_step while a tile shape was
+  // set by hand or is being timed
+  Tile* d_mtiles = nullptr;
+  size_t mtiles_cap = 0;
+  MultiPlan multi{};
+  uint32_t mbegin[4] = {};  // the tiles of multi.shape[i]: [mbegin[i], mbegin[i + 1])
+  void* spare = nullptr;
+  bool spare_asked = false;
+  bool one_step = false;
   hipGraphExec_t chain = nullptr;
   uint64_t chain_len = 0;
   int chain_res = -1;
@@ -1392,8 +1505,9 @@ struct lbm_batch {
 
 namespace {
 
-StepArgs member_args(const lbm_ctx* c) {
+StepArgs member_args(const lbm_ctx* c, void* f2) {
   StepArgs a{};
+  a.f2 = f2;
   a.f = c->f;
   a.flags = c->flags;
   a.ops = c->ops;
@@ -1411,6 +1525,7 @@ StepArgs member_args(const lbm_ctx* c) {
   a.Np = c->Np;
   a.periodic = c->periodic;
   a.status = c->status_d;
+  classify(c, a);
   return a;
 }
 
@@ -1433,16 +1548,49 @@ lbm_status build_tiles(lbm_batch* b) {
   std::vector<Tile> tiles;
   std::vector<uint32_t> begin(M + 1, 0);
   const int bx = b->shape.block, rows = b->shape.rows;
+  HIP_TRY(hipSetDevice(b->device));
+  // multi-step launches where every member's operators allow them
+  bool ok = !b->one_step;
+  uint64_t cells = 0;
+  size_t bytes = 0;
+  std::vector<size_t> at(M, 0);
+  for (uint32_t m = 0; m < M; ++m) {
+    ok = ok && multi_operators(b->members[m]);
+    if (b->active[m]) cells += b->members[m]->N;
+    at[m] = bytes;
+    bytes += (b->members[m]->fbytes() + 255) / 256 * 256;
+  }
+  if (ok && !b->spare_asked) {
+    b->spare_asked = true;
+    b->spare = spare_buffer(bytes);
+  }
+  ok = ok && b->spare;
+  b->multi = ok ? multi_plan(b->storage, cells) : MultiPlan{};
+  std::vector<Tile> mtiles;
+  for (int i = 0; i < b->multi.n; ++i) {
+    const MultiShape& sh = b->multi.shape[i];
+    b->mbegin[i] = uint32_t(mtiles.size());
+    for (uint32_t m = 0; m < M; ++m) {
+      if (!b->active[m]) continue;
+      const uint64_t tx = (b->members[m]->n[0] + sh.tx - 1) / sh.tx, ty = (b->members[m]->n[1] + sh.ty - 1) / sh.ty;
+      if (tx > 0xffff || ty > 0xffff) {  // beyond the tile record
+        b->multi.n = 0;
+        break;
+      }
+      for (uint32_t y = 0; y < ty; ++y)
+        for (uint32_t x = 0; x < tx; ++x) mtiles.push_back(Tile{m, x | (y << 16)});
+    }
+    b->mbegin[i + 1] = uint32_t(mtiles.size());
+  }
   for (uint32_t m = 0; m < M; ++m) {
     lbm_ctx* c = b->members[m];
-    args[m] = member_args(c);
+    args[m] = member_args(c, ok ? static_cast<char*>(b->spare) + at[m] : nullptr);
     begin[m] = uint32_t(tiles.size());
     if (!b->active[m]) continue;
     const uint64_t per = uint64_t(bx) * uint64_t(rows);
     for (uint64_t c0 = 0; c0 < c->N; c0 += per) tiles.push_back(Tile{m, uint32_t(c0)});
   }
   begin[M] = uint32_t(tiles.size());
-  HIP_TRY(hipSetDevice(b->device));
   HIP_TRY(hipStreamSynchronize(b->stream));
   if (tiles.size() > b->tiles_cap) {
     if (b->d_tiles) HIP_TRY(hipFree(b->d_tiles));
@@ -1452,6 +1600,15 @@ lbm_status build_tiles(lbm_batch* b) {
     HIP_TRY(hipMalloc((void**)&b->d_partial, b->tiles_cap * 2 * sizeof(double)));
   }
   b->ntiles = uint32_t(tiles.size());
+  if (mtiles.size() > b->mtiles_cap) {
+    if (b->d_mtiles) HIP_TRY(hipFree(b->d_mtiles));
+    b->d_mtiles = nullptr;
+    b->mtiles_cap = 0;
+    HIP_TRY(hipMalloc((void**)&b->d_mtiles, mtiles.size() * sizeof(Tile)));
+    b->mtiles_cap = mtiles.size();
+  }
+  if (!mtiles.empty())
+    HIP_TRY(hipMemcpyAsync(b->d_mtiles, mtiles.data(), mtiles.size() * sizeof(Tile), hipMemcpyHostToDevice, b->stream));
   if (!tiles.empty())
     HIP_TRY(hipMemcpyAsync(b->d_tiles, tiles.data(), tiles.size() * sizeof(Tile), hipMemcpyHostToDevice, b->stream));
   HIP_TRY(hipMemcpyAsync(b->d_members, args.data(), M * sizeof(StepArgs), hipMemcpyHostToDevice, b->stream));
@@ -1480,6 +1637,19 @@ BatchArgs batch_args(lbm_batch* b, uint32_t k, int write_macros) {
 lbm_status enqueue_chain(lbm_batch* b, uint64_t n, bool with_res) {
   int phase = b->phase;
   for (uint64_t k = 0; k < n; ++k) {
+    const uint64_t silent = n - k - 1;  // steps before the one that writes the macros
+    const MultiShape* sh = phase == 0 ? multi_fit(b->multi, with_res && silent > 0 ? silent - 1 : silent) : nullptr;
+    if (sh) {
+      const int i = int(sh - b->multi.shape);
+      for (int flip = 0; flip < 2; ++flip) {
+        BatchArgs a = batch_args(b, uint32_t(k) + uint32_t(flip * sh->steps), 0);
+        a.tiles = b->d_mtiles + b->mbegin[i];
+        a.ntiles = b->mbegin[i + 1] - b->mbegin[i];
+        HIP_TRY(launch_multi_batch(b->storage, *sh, a, flip, b->stream));
+      }
+      k += 2u * uint64_t(sh->steps) - 1;
+      continue;
+    }
     int wm = 0;
     if (k + 1 == n) wm = 1;
     if (with_res && k + 2 == n) wm = 2;
@@ -1590,7 +1760,8 @@ lbm_status lbm_batch_destroy(lbm_batch* b) {
   drop_chain(b);
   for (void* p : b->uprev) (void)hipFree(p);
   for (lbm_ctx* c : b->members) lbm_ctx_destroy(c);
-  void* ptrs[] = {b->d_members, b->d_tiles, b->d_tile_begin, b->d_uprev, b->d_partial, b->d_res, b->d_t0};
+  void* ptrs[] = {b->d_members, b->d_tiles, b->d_tile_begin, b->d_uprev, b->d_partial,
+                  b->d_res,     b->d_t0,    b->d_mtiles,     b->spare};
   for (void* p : ptrs)
     if (p) (void)hipFree(p);
   if (b->ev0) (void)hipEventDestroy(b->ev0);
@@ -1697,6 +1868,7 @@ lbm_status lbm_batch_set_tuning(lbm_batch* b, const lbm_batch_tuning* t) {
   b->shape.block = t->block;
   b->shape.rows = t->rows;
   b->shape.grid = t->grid;
+  b->one_step = true;  // every step in this shape
   b->tiles_dirty = true;
   return LBM_OK;
 }
@@ -1738,6 +1910,13 @@ lbm_status lbm_batch_autotune(lbm_batch* b, lbm_batch_tuning* chosen) {
   const BatchShape keep = b->shape;
   BatchShape best = keep;
   double best_ms = 1e30;
+  // the trials time the one-step launches' tiles; the chains keep their
+  // multi-step launches
+  struct Pin {
+    bool &flag, was;
+    ~Pin() { flag = was; }
+  } pin{b->one_step, b->one_step};
+  b->one_step = true;
   const int blocks[3] = {64, 128, 256}, rows_c[3] = {1, 2, 4}, grids[4] = {0, 4, 8, 16};
   for (int bi = 0; bi < 3; ++bi)
     for (int ri = 0; ri < 3; ++ri)
