@@ -12,12 +12,9 @@
 // over pixel ranges with a fixed-order reduction of the partial tiles, so
 // training is deterministic run to run.
 //
-// Block tile 128 (M) x 16*NC (N) x 32 (K), NC per layer so that the
-// layer's channel count is a whole number of tiles (up to 128 columns):
-// four 64-wide waves, each owning 32 rows x 16*NC columns = 2 x NC MFMA
-// 16x16 blocks.  A and B tiles are staged through two LDS buffers with the K
-// index contiguous, so that every MFMA operand is one 16-byte LDS read (rows
-// padded by 8 elements against bank conflicts); one barrier per K step.
+// A conv block takes 8 (or 4) x 16 pixels and 16*NC output channels, NC per
+// layer so that the layer's channel count is a whole number of tiles: the
+// pixels and their halo in LDS, the weights as ready MFMA fragments.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -34,6 +31,8 @@
 namespace lbmnet {
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 // Round-to-nearest-even FP32 -> bf16 bits (NaN kept quiet).
@@ -45,25 +44,32 @@ __host__ __device__ inline uint16_t f2bf(float f) {
 }
 __host__ __device__ inline float bf2f(uint16_t h) { return __builtin_bit_cast(float, uint32_t(h) << 16); }
 
+// Two of f2bf in one instruction (v_cvt_pk_bf16_f32 rounds to nearest even).
+__device__ inline uint32_t f2bf2(float a, float b) {
+  typedef float f32x2 __attribute__((ext_vector_type(2)));
+  typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+  return __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2{a, b}, bf16x2));
+}
+
 struct Act {  // element (pixel q, channel c) at p[q*ld + off + c]
   uint16_t* p;
   int ld, off;
 };
+// An activation lies kActPad elements into its allocation, behind zeros: what
+// a kernel reads for a pixel outside the image, by an offset from the same
+// base as the pixels (a 32-bit offset then serves both).
+constexpr int kActPad = 128;
+// Byte offsets from the allocation's start fit 32 bits.
+inline bool act_small(const Act& a, size_t pixels) { return (pixels * a.ld + kActPad) * 2 < (size_t(1) << 32); }
 
 constexpr int BM = 128, BK = 32, LK = BK + 8;
-// Conv K steps whose global loads are in flight across whole K steps (a
-// register ring of that many slots), per tile width.  0: the next step's
-// loads are issued at the start of a step and stored to LDS at its end.  2
-// for the 64-, 80- and 128-channel tiles (their conv 4-7% faster); the 32-
-// and 96-channel tiles are as fast or faster with 0 (the ring's registers
-// cost the 96-channel tile a wave per SIMD), and 4 or more slow every tile.
-constexpr int conv_prefetch(int nc) { return (nc == 4 || nc == 5 || nc == 8) ? 2 : 0; }
+
 
 struct ConvArgs {
   int B, H, W;
   int cin, cout;  // GEMM K = 9*cin, N = cout; both multiples of 8
   Act in, out;
-  const uint16_t* w;  // [9][cin][cout]
+  const uint4* w;  // weight fragments (k_wconvert)
   const float* bias;
   int bias_n;
   float* outf;  // FP32 result (ld outf_n, columns < outf_n) instead of out
@@ -77,6 +83,255 @@ __device__ inline uint4 load_tap(const Act& s, int H, int W, int b, int y, int x
   if (yy < 0 || yy >= H || xx < 0 || xx >= W) return make_uint4(0u, 0u, 0u, 0u);
   const size_t q = (size_t(b) * H + yy) * W + xx;
   return *reinterpret_cast<const uint4*>(s.p + q * s.ld + s.off + c);
+}
+
+// 16-channel tiles per conv block for N output channels: the widest block of
+// at most 128 channels that divides N (N = 8, the output layer, takes 32)
+__host__ __device__ inline int conv_nc(int N) {
+  const int nc[5] = {8, 6, 5, 4, 2};
+  for (int k = 0; k < 5; ++k)
+    if (N % (16 * nc[k]) == 0) return nc[k];
+  return 2;
+}
+// Weight fragments of a conv GEMM: per K step of 32 and 16-channel tile, the
+// 64 lanes' 16-byte MFMA operands in lane order, so a wavefront loads one as
+// 1 KiB in a row.  Lane l holds k = 8 (l / 16) .. + 7 of row l % 16.
+__host__ __device__ inline int conv_steps(int cin) { return (9 * cin + 31) / 32; }
+__host__ __device__ inline int conv_tiles(int N) {  // padded to whole blocks
+  const int nc = conv_nc(N);
+  return (N + 16 * nc - 1) / (16 * nc) * nc;
+}
+// The channel of row r of tile t.  Tiles go in pairs whose rows interleave by
+// four: lane group g of the result then holds the 8 consecutive channels
+// 8g .. 8g + 7 of the pair, one 16-byte store.
+__host__ __device__ inline int conv_channel(int nc, int t, int r) {
+  const int blk = t / nc, i = t - blk * nc, base = blk * nc * 16;
+  if ((i | 1) >= nc) return base + 16 * i + r;  // the last tile of an odd block
+  return base + 32 * (i / 2) + 8 * (r / 4) + 4 * (i & 1) + (r & 3);
+}
+
+constexpr int kPatchW = 18;  // 16 pixels and the halo
+
+
+// Forward convolution and data gradient: the implicit GEMM over the 3x3 taps.
+// A block takes 4*MT rows of 16 pixels of one image and 16*NC output
+// channels; the pixels with their halo go to LDS once, all channels (one read
+// of the activation instead of one per tap, one barrier instead of one per K
+// step), and the nine taps read them there, each 16-pixel operand at its own
+// shift.  Pixels lie 2*cin + 16 bytes apart.  The weights come as ready
+// fragments from L1/L2, so they need no LDS either.  A wavefront has MT rows of
+// pixels and all NC tiles: per K step MT operands from LDS and NC from L1 for
+// MT*NC MFMAs.  The weights are the first operand: a lane's results are then 8
+// consecutive channels of one pixel, stored as they are.  Batch of 16 images of
+// 256 x 256, per layer, against 128-pixel tiles gathered tap by tap through two
+// LDS buffers: 96 -> 32 channels 237 -> 110 us, 32 -> 32 79 -> 42 us, at 32 x 32
+// 96 -> 160 and 160 -> 160 channels 33 and 46 -> 16 and 22 us.  What bounds it
+// then: the many-channel layers the MFMA issue (96 -> 32: 58 GFLOP, 42 us at the
+// card's matrix-product rate) and LDS reads, the few-channel ones memory; the
+// input gradient of 96 channels at 256 x 256 (184 us, as before) the 400 MB of
+// its mask and result.
+// MODE 0: cin a multiple of 32 (a K step lies in one tap); 1: any cin (each
+// quarter of the lanes finds its own tap); 2: as 1, with the pixels read from
+// the activation (their patch would not fit LDS, or their offsets 32 bits).
+template <int NC, int MT, int MODE>
+__global__ __launch_bounds__(256) void k_conv(ConvArgs a) {
+  extern __shared__ u32x4 patch[];
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, g = lane >> 4, px = lane & 15;
+  const int tx = (a.W + 15) / 16, ty = (a.H + 4 * MT - 1) / (4 * MT);
+  const int bx = blockIdx.x % tx, by = blockIdx.x / tx % ty, b = blockIdx.x / (tx * ty);
+  const int x0 = bx * 16, y0 = by * 4 * MT;
+  const int c8 = a.cin / 8, sp = c8 + 1;  // pixel pitch in 16-byte units
+  const int nk = conv_steps(a.cin), nt = conv_tiles(a.cout), t0 = blockIdx.y * NC;
+  const int zat = c8;  // MODE 1: a chunk of zeros (the first pixel's padding)
+  if (MODE != 2) {
+    // straight to LDS, 1 KiB a wavefront and instruction, so that the whole
+    // patch is in flight at once and takes no registers; a wavefront loads
+    // whole patch rows, whose lanes keep their column and chunk
+    const int row = kPatchW * sp;
+    for (int i0 = 0; i0 < row; i0 += 64) {
+      const int i = i0 + lane, x = i / sp, c = i - x * sp;
+      const bool in = c < c8 && unsigned(x0 - 1 + x) < unsigned(a.W) && i < row;
+      const uint32_t o = uint32_t((x * a.in.ld + c * 8) * 2);
+      for (int r = wave; r < 4 * MT + 2; r += 4) {
+        u32x4* to = patch + r * row + i0;
+        if (in && unsigned(y0 - 1 + r) < unsigned(a.H)) {
+          const auto from = (const __attribute__((address_space(1))) char*)(
+              a.in.p + ((size_t(b) * a.H + (y0 - 1 + r)) * a.W + x0) * a.in.ld + a.in.off - a.in.ld);
+          __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(from + o),
+                                           (__attribute__((address_space(3))) void*)to, 16, 0, 0);
+        } else if (i < row) {
+          to[lane] = u32x4{0u, 0u, 0u, 0u};
+        }
+      }
+    }
+    __builtin_amdgcn_s_waitcnt(0);
+    __syncthreads();
+  }
+  // what the results will need of the layer's input, in flight under the MFMAs
+  constexpr int NP = (NC + 1) / 2;
+  const int x = x0 + px;
+  auto pixel = [&](int r) { return (size_t(b) * a.H + (y0 + wave * MT + r)) * a.W + x; };
+  auto inside = [&](int r) { return y0 + wave * MT + r < a.H && x < a.W; };
+  // a pair's first channel in this lane
+  auto channel = [&](int p) { return 16 * (t0 + 2 * p) + (2 * p + 1 < NC ? 8 : 4) * g; };
+  u32x4 mk[MT][NP];
+  if (a.mask.p) {
+    const auto mp = (const __attribute__((address_space(1))) uint16_t*)a.mask.p + a.mask.off;
+#pragma unroll
+    for (int r = 0; r < MT; ++r)
+#pragma unroll
+      for (int p = 0; p < NP; ++p) {
+        const auto at = mp + (inside(r) ? pixel(r) * a.mask.ld : size_t(0)) + (channel(p) < a.cout ? channel(p) : 0);
+        if (2 * p + 1 < NC) {
+          mk[r][p] = *(const __attribute__((address_space(1))) u32x4*)at;
+        } else {
+          const auto t = *(const __attribute__((address_space(1))) u32x2*)at;
+          mk[r][p] = u32x4{t.x, t.y, 0u, 0u};
+        }
+      }
+  }
+  f32x4 acc[MT][NC];
+#pragma unroll
+  for (int r = 0; r < MT; ++r)
+#pragma unroll
+    for (int c = 0; c < NC; ++c) acc[r][c] = f32x4{0.f, 0.f, 0.f, 0.f};
+  const auto wp = (const __attribute__((address_space(1))) u32x4*)a.w + size_t(t0) * 64 + lane;
+  const int base = (wave * MT * kPatchW + px) * sp + (MODE == 0 ? g : 0);
+  int tap = 0, c = 0;  // MODE 0: the K step's tap and first 8-channel chunk
+  auto mma = [&](const u32x4 (&w)[NC], const u32x4 (&p)[MT]) {
+#pragma unroll
+    for (int r = 0; r < MT; ++r)
+#pragma unroll
+      for (int n = 0; n < NC; ++n)
+        acc[r][n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, w[n]),
+                                                            __builtin_bit_cast(bf16x8, p[r]), acc[r][n], 0, 0, 0);
+  };
+  if constexpr (MODE == 0) {
+    // nk = 9 * cin / 32 is a multiple of 3: three K steps per turn, the
+    // weights of each loaded a whole turn ahead (the last turn's loads read
+    // the fragments' padding)
+    u32x4 wf[3][NC];
+#pragma unroll
+    for (int d = 0; d < 3; ++d)
+#pragma unroll
+      for (int n = 0; n < NC; ++n) wf[d][n] = wp[(d * nt + n) * 64];
+    for (int k = 0; k < nk; k += 3) {
+#pragma unroll
+      for (int d = 0; d < 3; ++d) {
+        u32x4 pf[MT];
+        const int off = base + (tap / 3 * kPatchW + tap % 3) * sp + c;
+#pragma unroll
+        for (int r = 0; r < MT; ++r) pf[r] = patch[off + r * kPatchW * sp];
+        c += 4;
+        if (c == c8) {
+          c = 0;
+          ++tap;
+        }
+        mma(wf[d], pf);
+#pragma unroll
+        for (int n = 0; n < NC; ++n) wf[d][n] = wp[size_t((k + 3 + d) * nt + n) * 64];
+      }
+    }
+  } else {
+    for (int k = 0; k < nk; ++k) {
+      u32x4 wf[NC], pf[MT];
+#pragma unroll
+      for (int n = 0; n < NC; ++n) wf[n] = wp[size_t(k * nt + n) * 64];
+      const int o = 4 * k + g, tp = o / c8, ch = o - tp * c8;  // this lane's tap and 8-channel chunk
+      const bool in = tp < 9;
+#pragma unroll
+      for (int r = 0; r < MT; ++r) {
+        if (MODE == 1) {
+          pf[r] = patch[in ? base + (r * kPatchW + tp / 3 * kPatchW + tp % 3) * sp + ch : zat];
+        } else {
+          const int y = y0 + wave * MT + r, x = x0 + px;
+          const uint4 v = (in && y < a.H && x < a.W) ? load_tap(a.in, a.H, a.W, b, y, x, tp, ch * 8)
+                                                     : make_uint4(0u, 0u, 0u, 0u);
+          pf[r] = u32x4{v.x, v.y, v.z, v.w};
+        }
+      }
+      mma(wf, pf);
+    }
+  }
+  // 8 channels of a pixel per lane and store
+#pragma unroll
+  for (int p = 0; p < NP; ++p) {
+    const bool pair = 2 * p + 1 < NC;
+    const int ch = channel(p);
+    if (ch >= a.cout) continue;
+    float bias[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) bias[j] = (a.bias && ch + j < a.bias_n && (pair || j < 4)) ? a.bias[ch + j] : 0.f;
+#pragma unroll
+    for (int r = 0; r < MT; ++r) {
+      if (!inside(r)) continue;
+      const size_t m = pixel(r);
+      float v[8];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        v[j] = j < 4 ? acc[r][2 * p][j] : (pair ? acc[r][pair ? 2 * p + 1 : 2 * p][j - 4] : 0.f);
+        if (a.bias) v[j] = v[j] + bias[j];
+        if (a.relu) v[j] = v[j] > 0.f ? v[j] : 0.f;
+      }
+      if (a.outf) {  // FP32 result (the output layer)
+#pragma unroll
+        for (int j = 0; j < 8; ++j)
+          if (ch + j < a.outf_n && (pair || j < 4)) a.outf[m * a.outf_n + ch + j] = v[j];
+        continue;
+      }
+      u32x4 w;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) w[j] = f2bf2(v[2 * j], v[2 * j + 1]);
+      if (a.mask.p) {  // zero where the layer input was not positive
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          if (!(bf2f(uint16_t(mk[r][p][j] & 0xffffu)) > 0.f)) w[j] &= 0xffff0000u;
+          if (!(bf2f(uint16_t(mk[r][p][j] >> 16)) > 0.f)) w[j] &= 0x0000ffffu;
+        }
+      }
+      const auto op = (__attribute__((address_space(1))) uint16_t*)a.out.p + m * a.out.ld + a.out.off + ch;
+      if (pair) *(__attribute__((address_space(1))) u32x4*)op = w;
+      else *(__attribute__((address_space(1))) u32x2*)op = u32x2{w[0], w[1]};
+    }
+  }
+}
+
+template <int NC, int MT>
+hipError_t launch_conv_t(const ConvArgs& a, size_t lds, hipStream_t s) {
+  const dim3 grid(a.B * ((a.H + 4 * MT - 1) / (4 * MT)) * ((a.W + 15) / 16), conv_tiles(a.cout) / NC);
+  if (lds > 160 * 1024 || !act_small(a.in, size_t(a.B) * a.H * a.W)) {
+    hipLaunchKernelGGL((k_conv<NC, MT, 2>), grid, dim3(256), 0, s, a);
+  } else if (a.cin % 32 == 0) {
+    hipLaunchKernelGGL((k_conv<NC, MT, 0>), grid, dim3(256), lds, s, a);
+  } else {
+    hipLaunchKernelGGL((k_conv<NC, MT, 1>), grid, dim3(256), lds, s, a);
+  }
+  return hipGetLastError();
+}
+
+template <int NC>
+hipError_t launch_conv_n(const ConvArgs& a, hipStream_t s) {
+  // Blocks of 8 x 16 pixels, unless their patch exceeds LDS or the chip has
+  // more CUs than there are such blocks: 4 x 16 there (64 x 64 images of a batch
+  // of 16, 160 -> 96 channels: 22 us, 19 us with the lower block).  16 x 16 pixels
+  // hold twice the accumulators and a patch that leaves fewer blocks on a CU:
+  // 94 us for 75 us at 128 x 128, 160 -> 64 channels.
+  auto lds = [&](int mt) { return size_t(((4 * mt + 2) * kPatchW) * (a.cin / 8 + 1) + 255) / 256 * 4096; };
+  auto blocks = [&](int mt) {
+    return size_t(a.B) * ((a.H + 4 * mt - 1) / (4 * mt)) * ((a.W + 15) / 16) * (conv_tiles(a.cout) / NC);
+  };
+  if (lds(2) <= 160 * 1024 && blocks(2) >= 256) return launch_conv_t<NC, 2>(a, lds(2), s);
+  return launch_conv_t<NC, 1>(a, lds(1), s);
+}
+
+hipError_t launch_conv(const ConvArgs& a, hipStream_t s) {
+  switch (conv_nc(a.cout)) {
+    case 8: return launch_conv_n<8>(a, s);
+    case 6: return launch_conv_n<6>(a, s);
+    case 5: return launch_conv_n<5>(a, s);
+    case 4: return launch_conv_n<4>(a, s);
+    default: return launch_conv_n<2>(a, s);
+  }
 }
 
 // A wavefront's 32 rows of the block tile against NC 16-column blocks of the
@@ -98,183 +353,12 @@ __device__ inline void mma_tile_n(const uint16_t* As, const uint16_t* Bs, int wa
   }
 }
 
-// Forward convolution and data gradient (implicit GEMM over 3x3 taps).
-// Block tile BM = 128 pixels x 16*NC output channels (NC chosen per layer so
-// the channel count is a whole number of tiles), K in steps of 32 through
-// two LDS buffers: the next step's A (gathered taps) and B (weights, stored
-// N-major with K contiguous, so both tiles go to LDS without transposing)
-// are loaded into registers while the current step's MFMAs run, then written
-// to the other buffer; one barrier per K step.
-template <int NC>
-__global__ __launch_bounds__(256) void k_conv(ConvArgs a) {
-  constexpr int BNc = 16 * NC;
-  constexpr int NB = (BNc * 4 + 255) / 256;  // B chunks of 8 per thread
-  constexpr int KP = conv_prefetch(NC);
-  constexpr int KS = KP > 0 ? KP : 1;  // ring slots
-  // the two tile buffers; after the K loop the same LDS holds the block's
-  // bf16 results for 16-byte stores (128 rows of BNc + 8 values)
-  constexpr int kTiles = 2 * BM * LK + 2 * BNc * LK, kOut = BM * (BNc + 8);
-  __shared__ __align__(16) uint16_t smem[kTiles > kOut ? kTiles : kOut];
-  uint16_t (*As)[BM * LK] = reinterpret_cast<uint16_t (*)[BM * LK]>(smem);
-  uint16_t (*Bs)[BNc * LK] = reinterpret_cast<uint16_t (*)[BNc * LK]>(smem + 2 * BM * LK);
-  const int M = a.B * a.H * a.W, K = 9 * a.cin, N = a.cout, HW = a.H * a.W;
-  const int m0 = blockIdx.x * BM, n0 = blockIdx.y * BNc;
-  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-  const int kc = (tid & 3) * 8;
-  int rb[2], ry[2], rx[2];
-  bool rv[2];
-#pragma unroll
-  for (int j = 0; j < 2; ++j) {
-    const int m = m0 + ((tid + 256 * j) >> 2);
-    rv[j] = m < M;
-    const int mm = rv[j] ? m : 0;
-    rb[j] = mm / HW;
-    const int r = mm - rb[j] * HW;
-    ry[j] = r / a.W;
-    rx[j] = r - ry[j] * a.W;
-  }
-  // slot q of the ring holds the A and B chunks of one K step from its load
-  // to its LDS store
-  uint4 ra[KS][2], rw[KS][NB];
-  auto gload = [&](int q, int k0) {
-    const int kk = k0 + kc;
-    int tap = 0, c = 0;
-    if (kk < K) {
-      tap = kk / a.cin;
-      c = kk - tap * a.cin;
-    }
-#pragma unroll
-    for (int j = 0; j < 2; ++j)
-      ra[q][j] = (rv[j] && kk < K) ? load_tap(a.in, a.H, a.W, rb[j], ry[j], rx[j], tap, c) : make_uint4(0u, 0u, 0u, 0u);
-#pragma unroll
-    for (int qq = 0; qq < NB; ++qq) {
-      const int i = tid + 256 * qq;
-      const int n = n0 + (i >> 2), k = k0 + (i & 3) * 8;
-      rw[q][qq] = (i < BNc * 4 && n < N && k < K) ? *reinterpret_cast<const uint4*>(a.w + size_t(n) * K + k)
-                                                   : make_uint4(0u, 0u, 0u, 0u);
-    }
-  };
-  auto sstore = [&](int buf, int q) {
-#pragma unroll
-    for (int j = 0; j < 2; ++j) *reinterpret_cast<uint4*>(&As[buf][((tid + 256 * j) >> 2) * LK + kc]) = ra[q][j];
-#pragma unroll
-    for (int qq = 0; qq < NB; ++qq) {
-      const int i = tid + 256 * qq;
-      if (i < BNc * 4) *reinterpret_cast<uint4*>(&Bs[buf][(i >> 2) * LK + (i & 3) * 8]) = rw[q][qq];
-    }
-  };
-  f32x4 acc[2][NC];
-#pragma unroll
-  for (int r = 0; r < 2; ++r)
-#pragma unroll
-    for (int c = 0; c < NC; ++c) acc[r][c] = f32x4{0.f, 0.f, 0.f, 0.f};
-  const int nk = (K + BK - 1) / BK;
-  gload(0, 0);
-  sstore(0, 0);
-#pragma unroll
-  for (int j = 1; j <= KP; ++j)
-    if (j < nk) gload(j % KS, j * BK);
-  __syncthreads();
-  if constexpr (KP == 0) {
-    for (int kt = 0; kt < nk; ++kt) {
-      if (kt + 1 < nk) gload(0, (kt + 1) * BK);
-      mma_tile_n<NC>(As[kt & 1], Bs[kt & 1], wave, lane, acc);
-      if (kt + 1 < nk) sstore((kt + 1) & 1, 0);  // read by no wave since the last barrier
-      __syncthreads();
-    }
-  } else {
-    // step kt: MFMAs on LDS buffer kt & 1; step kt + 1 from the ring into
-    // the other buffer (read by no wave since the last barrier); its slot
-    // then takes the loads of step kt + 1 + KP (slots are compile-time
-    // indices)
-    for (int kt0 = 0; kt0 < nk; kt0 += KS) {
-#pragma unroll
-      for (int j = 0; j < KS; ++j) {
-        const int kt = kt0 + j;
-        if (kt < nk) {
-          mma_tile_n<NC>(As[kt & 1], Bs[kt & 1], wave, lane, acc);
-          if (kt + 1 < nk) sstore((kt + 1) & 1, (j + 1) % KS);
-          if (kt + 1 + KP < nk) gload((j + 1) % KS, (kt + 1 + KP) * BK);
-          __syncthreads();
-        }
-      }
-    }
-  }
-  if (a.outf) {  // FP32 result (the output layer)
-#pragma unroll
-    for (int r = 0; r < 2; ++r)
-#pragma unroll
-      for (int c = 0; c < NC; ++c)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          const int m = m0 + wave * 32 + r * 16 + (lane >> 4) * 4 + j;
-          const int n = n0 + c * 16 + (lane & 15);
-          if (m >= M || n >= a.outf_n) continue;
-          float v = acc[r][c][j];
-          if (a.bias && n < a.bias_n) v = v + a.bias[n];
-          if (a.relu) v = v > 0.f ? v : 0.f;
-          a.outf[size_t(m) * a.outf_n + n] = v;
-        }
-    return;
-  }
-  // bias and ReLU into the LDS tile (the K loop ended with a barrier) ...
-  constexpr int OP = BNc + 8;
-#pragma unroll
-  for (int r = 0; r < 2; ++r)
-#pragma unroll
-    for (int c = 0; c < NC; ++c)
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const int row = wave * 32 + r * 16 + (lane >> 4) * 4 + j, col = c * 16 + (lane & 15);
-        const int n = n0 + col;
-        float v = acc[r][c][j];
-        if (a.bias && n < a.bias_n) v = v + a.bias[n];
-        if (a.relu) v = v > 0.f ? v : 0.f;
-        smem[row * OP + col] = f2bf(v);
-      }
-  __syncthreads();
-  // ... then 8 channels per 16-byte store, with the input-gradient mask
-  // (zero where the layer input was not positive) applied per element
-  constexpr int CH = BNc / 8;
-  for (int t = tid; t < BM * CH; t += 256) {
-    const int row = t / CH, ch = t - row * CH;
-    const int m = m0 + row, n = n0 + ch * 8;
-    if (m >= M || n >= N) continue;
-    uint4 v = *reinterpret_cast<const uint4*>(&smem[row * OP + ch * 8]);
-    if (a.mask.p) {
-      const uint4 mk = *reinterpret_cast<const uint4*>(a.mask.p + size_t(m) * a.mask.ld + a.mask.off + n);
-      uint32_t w[4] = {v.x, v.y, v.z, v.w};
-      const uint32_t mw[4] = {mk.x, mk.y, mk.z, mk.w};
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        if (!(bf2f(uint16_t(mw[q] & 0xffffu)) > 0.f)) w[q] &= 0xffff0000u;
-        if (!(bf2f(uint16_t(mw[q] >> 16)) > 0.f)) w[q] &= 0x0000ffffu;
-      }
-      v = make_uint4(w[0], w[1], w[2], w[3]);
-    }
-    *reinterpret_cast<uint4*>(a.out.p + size_t(m) * a.out.ld + a.out.off + n) = v;
-  }
-}
-
-// 16-column blocks per conv tile for N output channels: the widest tile of
-// at most 128 channels that divides N (N = 8, the output layer, takes 32)
-int conv_nc(int N) {
+// 16-column blocks per weight-gradient tile for N output channels: the widest
+// tile of at most 128 channels that divides N (N = 8 takes 32)
+int wgrad_nc(int N) {
   for (int nc : {8, 6, 5, 4, 2})
     if (N % (16 * nc) == 0) return nc;
   return 2;
-}
-
-hipError_t launch_conv(const ConvArgs& a, hipStream_t s) {
-  const int M = a.B * a.H * a.W, nc = conv_nc(a.cout);
-  const dim3 grid((M + BM - 1) / BM, (a.cout + 16 * nc - 1) / (16 * nc));
-  switch (nc) {
-    case 8: hipLaunchKernelGGL(k_conv<8>, grid, dim3(256), 0, s, a); break;
-    case 6: hipLaunchKernelGGL(k_conv<6>, grid, dim3(256), 0, s, a); break;
-    case 5: hipLaunchKernelGGL(k_conv<5>, grid, dim3(256), 0, s, a); break;
-    case 4: hipLaunchKernelGGL(k_conv<4>, grid, dim3(256), 0, s, a); break;
-    default: hipLaunchKernelGGL(k_conv<2>, grid, dim3(256), 0, s, a); break;
-  }
-  return hipGetLastError();
 }
 
 struct WgradArgs {
@@ -399,17 +483,171 @@ __global__ __launch_bounds__(256) void k_wgrad(WgradArgs a) {
       }
 }
 
-hipError_t launch_wgrad(const WgradArgs& a, int splits, hipStream_t s) {
-  const int nc = conv_nc(a.cout);
-  const dim3 grid((9 * a.cin + 8 + BM - 1) / BM, (a.cout + 16 * nc - 1) / (16 * nc), splits);
-  switch (nc) {
-    case 8: hipLaunchKernelGGL(k_wgrad<8>, grid, dim3(256), 0, s, a); break;
-    case 6: hipLaunchKernelGGL(k_wgrad<6>, grid, dim3(256), 0, s, a); break;
-    case 5: hipLaunchKernelGGL(k_wgrad<5>, grid, dim3(256), 0, s, a); break;
-    case 4: hipLaunchKernelGGL(k_wgrad<4>, grid, dim3(256), 0, s, a); break;
-    default: hipLaunchKernelGGL(k_wgrad<2>, grid, dim3(256), 0, s, a); break;
+// The same partial tiles where image rows are a multiple of 32 pixels, so that a
+// K step lies in one row.  A block takes one split, the three taps of one dy,
+// 32 input channels and 16*NC output channels; per K step the input's 32
+// pixels with one more on either side serve the three taps.  Both operands go
+// to LDS as they lie in memory (pixel by pixel, straight from the loads) and are
+// transposed on the way out (ds_read_b64_tr_b16: 16 lanes read 4 pixels x 16
+// channels and each gets the 4 pixels of its channel); the pixel pitches are odd
+// multiples of 32 bytes, so the 4 pixels of a read lie in different banks.
+// (That transposing write, 32 bits at a time, is most of k_wgrad's time.)
+// Two buffers of kWgSteps K steps: the loads of one are in flight under the
+// MFMAs of the other.  Where a K step lies is scalar arithmetic; a load costs
+// its thread an add and a select (with addresses worked out per thread and
+// load, their arithmetic bound the kernel).  Of the 6 x NC result tiles a
+// wavefront has 3 x NC/2.  The K steps and their pixels are k_wgrad's, so the
+// partial sums are its bits.
+constexpr int kWgSteps = 2;
+template <int NC>
+__global__ __launch_bounds__(256) void k_wgrad32(WgradArgs a, int splits) {
+  constexpr int PA = 6, PB = (NC | 1) * 2;    // pixel pitch in 16-byte chunks
+  constexpr int CA = 34 * PA, CS = CA + 32 * PB;  // chunks of a K step: of the input, of both
+  constexpr int NT = (CS + 255) / 256, NH = (NC + 1) / 2;
+  __shared__ u32x4 buf[2][kWgSteps][CS];
+  const int M = a.B * a.H * a.W, N = a.cout, Mx = 9 * a.cin + 8;
+  // the blocks of a split read the same pixels: all of them on one XCD (blocks
+  // go round the 8 XCDs in turn), whose L2 then reads them once
+  const int cblocks = (a.cin + 31) / 32, per = 3 * cblocks * ((N + 16 * NC - 1) / (16 * NC));
+  const int turn = blockIdx.x / 8, s = turn / per * 8 + int(blockIdx.x) % 8, part = turn % per;
+  if (s >= splits) return;  // (the splits rounded up to the XCDs)
+  const int dy = part % 3, c0 = part / 3 % cblocks * 32, n0 = part / 3 / cblocks * 16 * NC;
+  const int p0 = s * a.chunk, p1 = min(p0 + a.chunk, M), nk = p1 > p0 ? (p1 - p0 + 31) / 32 : 0;
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, g = lane >> 4, j = lane & 15;
+  // This thread's chunks of a K step: byte offset in the first step from the
+  // allocation's start, and the cases in which there is nothing to load (a
+  // zero is then read): never mind the step (channels beyond the layer's,
+  // padding of the pitch), the row above or below the image, the pixel left or
+  // right of it.
+  constexpr uint32_t kNever = 1, kRow = 2, kLeft = 4, kRight = 8;
+  using GC = const __attribute__((address_space(1))) char;
+  uint32_t off[NT], gone[NT], adv[NT];
+  bool is_a[NT];
+#pragma unroll
+  for (int t = 0; t < NT; ++t) {
+    const int i = tid + 256 * t;
+    is_a[t] = i < CA;
+    const int px = is_a[t] ? i / PA : (i - CA) / PB, ch = is_a[t] ? i - px * PA : i - CA - px * PB;
+    const int c = (is_a[t] ? c0 : n0) + ch * 8;
+    const bool ok = i < CS && ch < (is_a[t] ? 4 : 2 * NC) && c < (is_a[t] ? a.cin : N);
+    gone[t] = !ok ? kNever : (!is_a[t] ? 0u : kRow | (px == 0 ? kLeft : 0u) | (px == 33 ? kRight : 0u));
+    const int ld = is_a[t] ? a.in.ld : a.dpre.ld;
+    const long long at = p0 + px + (is_a[t] ? (long long)(dy - 1) * a.W - 1 : 0ll);
+    off[t] = uint32_t((at * ld + (is_a[t] ? a.in.off : a.dpre.off) + c + kActPad) * 2);
+    adv[t] = 64u * uint32_t(ld);
   }
+  GC* in0 = (GC*)(a.in.p - kActPad);
+  GC* dp0 = (GC*)(a.dpre.p - kActPad);
+  int x = p0 % a.W, y = p0 / a.W % a.H, left = nk;  // the next K step to load, and how many there are
+  auto load = [&](int b) {
+#pragma unroll
+    for (int ks = 0; ks < kWgSteps; ++ks) {
+      if (left-- <= 0) break;
+      const uint32_t now = kNever | (unsigned(y + dy - 1) < unsigned(a.H) ? 0u : kRow) | (x == 0 ? kLeft : 0u) |
+                           (x + 32 == a.W ? kRight : 0u);
+#pragma unroll
+      for (int t = 0; t < NT; ++t) {
+        const uint32_t o = (gone[t] & now) ? 0u : off[t];
+        if (256 * (t + 1) <= CS || tid + 256 * t < CS)
+          __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)((is_a[t] ? in0 : dp0) + o),
+                                           (__attribute__((address_space(3))) void*)(&buf[b][ks][256 * t + wave * 64]),
+                                           16, 0, 0);
+        off[t] += adv[t];
+      }
+      x += 32;
+      if (x == a.W) {
+        x = 0;
+        if (++y == a.H) y = 0;
+      }
+    }
+  };
+  typedef short s16x4 __attribute__((ext_vector_type(4)));
+  using L4 = __attribute__((address_space(3))) s16x4;
+  // 8 pixels of a 16-channel operand: at, the lane's address of the first four
+  auto frag = [&](const uint16_t* at, int pitch) {
+    const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((L4*)at);
+    const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((L4*)(at + 4 * pitch * 8));
+    return __builtin_bit_cast(bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+  };
+  const int wm = wave & 1, wn = wave >> 1;
+  const bool bias = dy == 1 && c0 == 0 && wm == 1;  // row 9*cin: ones against dpre
+  f32x4 acc[3][NH], accb[NH];
+#pragma unroll
+  for (int n = 0; n < NH; ++n) {
+    accb[n] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int i = 0; i < 3; ++i) acc[i][n] = f32x4{0.f, 0.f, 0.f, 0.f};
+  }
+  const uint32_t one = j == 0 ? 0x3f803f80u : 0u;
+  const bf16x8 ones = __builtin_bit_cast(bf16x8, u32x4{one, one, one, one});
+  if (nk > 0) load(0);
+  for (int k0 = 0; k0 < nk; k0 += kWgSteps) {
+    const int b = (k0 / kWgSteps) & 1;
+    __builtin_amdgcn_s_waitcnt(0);
+    __syncthreads();  // this buffer has arrived; no wave reads the other one any more
+    if (k0 + kWgSteps < nk) load(b ^ 1);
+#pragma unroll
+    for (int ks = 0; ks < kWgSteps; ++ks) {
+      if (k0 + ks >= nk) break;
+      const uint16_t* lds = reinterpret_cast<const uint16_t*>(buf[b][ks]);
+      bf16x8 af[3], bf[NH];
+#pragma unroll
+      for (int i = 0; i < 3; ++i) {
+        const int tile = wm * 3 + i;  // tap dx = tile / 2, channels 16 (tile % 2) ..
+        af[i] = frag(lds + (8 * g + (j >> 2) + tile / 2) * PA * 8 + (tile & 1) * 16 + (j & 3) * 4, PA);
+      }
+#pragma unroll
+      for (int n = 0; n < NH; ++n)
+        if (wn * NH + n < NC)
+          bf[n] = frag(lds + CA * 8 + (8 * g + (j >> 2)) * PB * 8 + (wn * NH + n) * 16 + (j & 3) * 4, PB);
+#pragma unroll
+      for (int n = 0; n < NH; ++n) {
+        if (wn * NH + n >= NC) continue;
+#pragma unroll
+        for (int i = 0; i < 3; ++i) acc[i][n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bf[n], af[i], acc[i][n], 0, 0, 0);
+        if (bias) accb[n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bf[n], ones, accb[n], 0, 0, 0);
+      }
+    }
+  }
+  float* out = a.partial + size_t(s) * Mx * N;
+#pragma unroll
+  for (int n = 0; n < NH; ++n) {
+    const int col = n0 + (wn * NH + n) * 16 + g * 4;
+    if (wn * NH + n >= NC || col >= N) continue;
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+      const int tile = wm * 3 + i, c = c0 + (tile & 1) * 16 + j;
+      if (c < a.cin)
+        *reinterpret_cast<f32x4*>(out + size_t((dy * 3 + tile / 2) * a.cin + c) * N + col) = acc[i][n];
+    }
+    if (bias && j == 0) *reinterpret_cast<f32x4*>(out + size_t(9 * a.cin) * N + col) = accb[n];
+  }
+}
+
+template <int NC>
+hipError_t launch_wgrad_n(const WgradArgs& a, int splits, hipStream_t s) {
+  const int cols = (a.cout + 16 * NC - 1) / (16 * NC);
+  const size_t px = size_t(a.B) * a.H * a.W;
+  // Fewer channels than its 32 leave k_wgrad32's tiles mostly empty: 49 us for 41
+  // at 256 x 256 from 8 channels.  From 32 on it is the faster one there (96 -> 32
+  // channels 300 -> 167 us, 32 -> 32 128 -> 71 us, 32 -> 3 110 -> 57 us) and about
+  // even where rows are one K step long (160 channels at 32 x 32: 27 us both).
+  if (a.cin > 16 && a.W % 32 == 0 && act_small(a.in, px) && act_small(a.dpre, px))
+    hipLaunchKernelGGL(k_wgrad32<NC>, dim3((splits + 7) / 8 * 8 * 3 * ((a.cin + 31) / 32) * cols), dim3(256), 0, s, a,
+                       splits);
+  else
+    hipLaunchKernelGGL(k_wgrad<NC>, dim3((9 * a.cin + 8 + BM - 1) / BM, cols, splits), dim3(256), 0, s, a);
   return hipGetLastError();
+}
+
+hipError_t launch_wgrad(const WgradArgs& a, int splits, hipStream_t s) {
+  switch (wgrad_nc(a.cout)) {
+    case 8: return launch_wgrad_n<8>(a, splits, s);
+    case 6: return launch_wgrad_n<6>(a, splits, s);
+    case 5: return launch_wgrad_n<5>(a, splits, s);
+    case 4: return launch_wgrad_n<4>(a, splits, s);
+    default: return launch_wgrad_n<2>(a, splits, s);
+  }
 }
 
 // grad[m*cr + n] = sum_s partial[s][m][n] for m <= 9*cin, n < cr (the
@@ -456,7 +694,7 @@ __device__ inline void ld8(const uint16_t* p, float (&f)[8]) {
 __device__ inline void st8(uint16_t* p, const float (&f)[8]) {
   uint32_t w[4];
 #pragma unroll
-  for (int t = 0; t < 4; ++t) w[t] = uint32_t(f2bf(f[2 * t])) | (uint32_t(f2bf(f[2 * t + 1])) << 16);
+  for (int t = 0; t < 4; ++t) w[t] = f2bf2(f[2 * t], f[2 * t + 1]);
   *reinterpret_cast<uint4*>(p) = make_uint4(w[0], w[1], w[2], w[3]);
 }
 
@@ -601,16 +839,42 @@ __global__ void k_adam(float* w, const float* g, float* m1, float* m2, size_t n,
   w[i] = w[i] - lr * (a / c1) / (sqrtf(b / c2) + eps);
 }
 
-// FP32 master [9][cin][cr] -> the bf16 B operands of the conv GEMMs, N-major
-// with K contiguous: forward W[co][tap*cin + ci], data gradient
-// Wt[ci][(8 - tap)*cpad + co] (taps flipped).
-__global__ void k_wconvert(const float* wm, int cin, int cr, int cpad, uint16_t* wb, uint16_t* wt) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= 9 * cin * cpad) return;
-  const int co = i % cpad, ci = (i / cpad) % cin, tap = i / (cpad * cin);
-  const uint16_t v = co < cr ? f2bf(wm[(size_t(tap) * cin + ci) * cr + co]) : uint16_t(0);
-  wb[size_t(co) * (9 * cin) + tap * cin + ci] = v;
-  wt[size_t(ci) * (9 * cpad) + (8 - tap) * cpad + co] = v;
+// FP32 master [9][cin][cr] -> the bf16 weight fragments of the conv GEMMs:
+// forward (K = taps x cin, N = cpad) and data gradient (taps flipped, K = taps
+// x cpad, N = cin).  One launch for all layers.
+struct WconvLayer {
+  const float* wm;
+  uint16_t *wb, *wt;
+  int cin, cr, cpad;
+  size_t end;  // of this layer's elements in the launch
+};
+struct WconvArgs {
+  WconvLayer layer[12];
+};
+__host__ __device__ inline size_t conv_elements(int cin, int N) {
+  return size_t(conv_steps(cin)) * conv_tiles(N) * 512;
+}
+__global__ void k_wconvert(WconvArgs a) {
+  const size_t step = size_t(gridDim.x) * 256;
+  for (size_t i = size_t(blockIdx.x) * 256 + threadIdx.x; i < a.layer[11].end; i += step) {
+    int k = 0;
+    while (i >= a.layer[k].end) ++k;
+    const WconvLayer& L = a.layer[k];
+    size_t e = i - (k > 0 ? a.layer[k - 1].end : 0);
+    const size_t nf = conv_elements(L.cin, L.cpad);
+    const bool fwd = e < nf;
+    if (!fwd) e -= nf;
+    const int ci = fwd ? L.cin : L.cpad, N = fwd ? L.cpad : L.cin, nt = conv_tiles(N);
+    const int lane = int(e >> 3) & 63, frag = int(e >> 9), t = frag % nt;
+    const int kk = frag / nt * 32 + (lane >> 4) * 8 + int(e & 7), tap = kk / ci, c = kk - tap * ci;
+    const int n = conv_channel(conv_nc(N), t, lane & 15);
+    uint16_t v = 0;
+    if (tap < 9 && n < N) {
+      const int in = fwd ? c : n, out = fwd ? n : c;
+      if (out < L.cr) v = f2bf(L.wm[(size_t(fwd ? tap : 8 - tap) * L.cin + in) * L.cr + out]);
+    }
+    (fwd ? L.wb : L.wt)[e] = v;
+  }
 }
 
 // In-place standardisation of stored targets: t = (t - mu) / sd.
@@ -730,6 +994,16 @@ lbm_status dalloc(T** p, size_t count) {
   return LBM_OK;
 }
 
+lbm_status aalloc(uint16_t** p, size_t count) {
+  const lbm_status s = dalloc(p, count + kActPad);
+  if (s != LBM_OK) return s;
+  *p += kActPad;
+  return LBM_OK;
+}
+void afree(uint16_t* p) {
+  if (p) (void)hipFree(p - kActPad);
+}
+
 void build_layers(lbm_net* n) {
   const int* w = n->cfg.widths;
   struct Spec {
@@ -767,7 +1041,7 @@ Act act(uint16_t* p, int ld, int off = 0) { return Act{p, ld, off}; }
 constexpr int kWgradBlocks = LBMNET_WGRAD_BLOCKS;
 void wgrad_shape(const lbm_net* n, const Layer& L, int B, int& splits, int& chunk) {
   const int M = B * H_(n, L.level) * W_(n, L.level);
-  const int bn = 16 * conv_nc(L.cpad);
+  const int bn = 16 * wgrad_nc(L.cpad);
   const int tiles = ((9 * L.cin + 8 + BM - 1) / BM) * ((L.cpad + bn - 1) / bn);
   splits = std::max(1, std::min(kWgradBlocks / std::max(1, tiles), (M + 255) / 256));
   chunk = ((M + splits - 1) / splits + BK - 1) / BK * BK;
@@ -784,7 +1058,7 @@ lbm_status conv(lbm_net* n, int li, int B, Act in, Act out, float* outf) {
   a.cout = L.cpad;
   a.in = in;
   a.out = out;
-  a.w = L.wb;
+  a.w = reinterpret_cast<const uint4*>(L.wb);
   a.bias = n->w + L.b_off;
   a.bias_n = L.cr;
   a.outf = outf;
@@ -818,7 +1092,7 @@ lbm_status conv_bwd(lbm_net* n, int li, int B, Act in, Act dpre, Act dx, bool ma
     a.cout = L.cin;
     a.in = dpre;
     a.out = dx;
-    a.w = L.wt;
+    a.w = reinterpret_cast<const uint4*>(L.wt);
     a.bias = nullptr;
     a.bias_n = 0;
     a.outf = nullptr;
@@ -930,11 +1204,15 @@ lbm_status backward(lbm_net* n, int B) {
 }
 
 lbm_status refresh_weights(lbm_net* n) {
-  for (Layer& L : n->layers) {
-    hipLaunchKernelGGL(k_wconvert, dim3(blocks_for(size_t(9) * L.cin * L.cpad)), dim3(256), 0, n->stream,
-                       n->w + L.w_off, L.cin, L.cr, L.cpad, L.wb, L.wt);
-    NET_TRY(hipGetLastError());
+  WconvArgs a{};
+  size_t end = 0;
+  for (int k = 0; k < 12; ++k) {
+    const Layer& L = n->layers[k];
+    end += conv_elements(L.cin, L.cpad) + conv_elements(L.cpad, L.cin);
+    a.layer[k] = WconvLayer{n->w + L.w_off, L.wb, L.wt, L.cin, L.cr, L.cpad, end};
   }
+  hipLaunchKernelGGL(k_wconvert, dim3(unsigned(std::min<size_t>(blocks_for(end), 1 << 20))), dim3(256), 0, n->stream, a);
+  NET_TRY(hipGetLastError());
   return LBM_OK;
 }
 
@@ -996,22 +1274,14 @@ void free_all(lbm_net* n) {
     (void)hipFree(L.wb);
     (void)hipFree(L.wt);
   }
-  void* ps[] = {n->w,      n->g,       n->m1,      n->m2,       n->x,       n->bott,      n->gbott, n->gy,
-                n->y,      n->t,       n->msk,     n->partial,  n->lpartial, n->dloss,  n->dlosses,
-                n->didx,   n->xs,      n->ts,      n->ms};
+  void* ps[] = {n->w,        n->g,     n->m1,      n->m2,   n->y,  n->t,  n->msk, n->partial,
+                n->lpartial, n->dloss, n->dlosses, n->didx, n->xs, n->ts, n->ms};
   for (void* p : ps) (void)hipFree(p);
-  for (int l = 0; l < 4; ++l) {
-    (void)hipFree(n->a[l]);
-    (void)hipFree(n->ga[l]);
-    (void)hipFree(n->pool[l]);
-    (void)hipFree(n->gpool[l]);
-  }
-  for (int l = 0; l < 3; ++l) {
-    (void)hipFree(n->cat[l]);
-    (void)hipFree(n->gcat[l]);
-    (void)hipFree(n->dec[l]);
-    (void)hipFree(n->gdec[l]);
-  }
+  for (uint16_t* p : {n->x, n->bott, n->gbott, n->gy}) afree(p);
+  for (int l = 0; l < 4; ++l)
+    for (uint16_t* p : {n->a[l], n->ga[l], n->pool[l], n->gpool[l]}) afree(p);
+  for (int l = 0; l < 3; ++l)
+    for (uint16_t* p : {n->cat[l], n->gcat[l], n->dec[l], n->gdec[l]}) afree(p);
   if (n->ev0) (void)hipEventDestroy(n->ev0);
   if (n->ev1) (void)hipEventDestroy(n->ev1);
   if (n->stream) (void)hipStreamDestroy(n->stream);
@@ -1030,28 +1300,29 @@ lbm_status create_impl(lbm_net* n) {
   NS(dalloc(&n->m1, n->nparam));
   NS(dalloc(&n->m2, n->nparam));
   for (Layer& L : n->layers) {
-    NS(dalloc(&L.wb, size_t(9) * L.cin * L.cpad));
-    NS(dalloc(&L.wt, size_t(9) * L.cin * L.cpad));
+    // (three K steps of padding: the conv's last turn loads a turn ahead)
+    NS(dalloc(&L.wb, conv_elements(L.cin, L.cpad) + 3 * 512 * size_t(conv_tiles(L.cpad))));
+    NS(dalloc(&L.wt, conv_elements(L.cpad, L.cin) + 3 * 512 * size_t(conv_tiles(L.cin))));
   }
   const int cw[3] = {w[1] + w[0], w[2] + w[1], w[3] + w[2]};
-  NS(dalloc(&n->x, level_pixels(n, 0) * 8));
+  NS(aalloc(&n->x, level_pixels(n, 0) * 8));
   for (int l = 0; l < 4; ++l) {
-    NS(dalloc(&n->a[l], level_pixels(n, l) * w[l]));
-    NS(dalloc(&n->ga[l], level_pixels(n, l) * w[l]));
+    NS(aalloc(&n->a[l], level_pixels(n, l) * w[l]));
+    NS(aalloc(&n->ga[l], level_pixels(n, l) * w[l]));
     if (l > 0) {
-      NS(dalloc(&n->pool[l], level_pixels(n, l) * w[l - 1]));
-      NS(dalloc(&n->gpool[l], level_pixels(n, l) * w[l - 1]));
+      NS(aalloc(&n->pool[l], level_pixels(n, l) * w[l - 1]));
+      NS(aalloc(&n->gpool[l], level_pixels(n, l) * w[l - 1]));
     }
   }
   for (int l = 0; l < 3; ++l) {
-    NS(dalloc(&n->cat[l], level_pixels(n, l) * cw[l]));
-    NS(dalloc(&n->gcat[l], level_pixels(n, l) * cw[l]));
-    NS(dalloc(&n->dec[l], level_pixels(n, l) * w[l]));
-    NS(dalloc(&n->gdec[l], level_pixels(n, l) * w[l]));
+    NS(aalloc(&n->cat[l], level_pixels(n, l) * cw[l]));
+    NS(aalloc(&n->gcat[l], level_pixels(n, l) * cw[l]));
+    NS(aalloc(&n->dec[l], level_pixels(n, l) * w[l]));
+    NS(aalloc(&n->gdec[l], level_pixels(n, l) * w[l]));
   }
-  NS(dalloc(&n->bott, level_pixels(n, 3) * w[3]));
-  NS(dalloc(&n->gbott, level_pixels(n, 3) * w[3]));
-  NS(dalloc(&n->gy, level_pixels(n, 0) * 8));
+  NS(aalloc(&n->bott, level_pixels(n, 3) * w[3]));
+  NS(aalloc(&n->gbott, level_pixels(n, 3) * w[3]));
+  NS(aalloc(&n->gy, level_pixels(n, 0) * 8));
   NS(dalloc(&n->y, level_pixels(n, 0) * 3));
   NS(dalloc(&n->t, level_pixels(n, 0) * 3));
   NS(dalloc(&n->msk, level_pixels(n, 0)));
