@@ -107,11 +107,6 @@ __global__ void k_pack(S* __restrict__ f, const double* __restrict__ in, Geometr
 }
 
 template <class T>
-__global__ void k_to_double(const T* __restrict__ a, double* __restrict__ b, size_t n) {
-  const size_t i = size_t(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (i < n) b[i] = double(a[i]);
-}
-template <class T>
 __global__ void k_from_double(T* __restrict__ a, const double* __restrict__ b, size_t n) {
   const size_t i = size_t(blockIdx.x) * blockDim.x + threadIdx.x;
   if (i < n) a[i] = T(b[i]);
@@ -172,15 +167,6 @@ hipError_t pack_populations(int lattice, int storage, void* f, const double* in,
   return hipErrorInvalidValue;
 }
 
-hipError_t field_to_double(bool is_double, const void* a, double* b, size_t n, hipStream_t s) {
-  if (n == 0) return hipSuccess;
-  dim3 bl(256), gr(unsigned((n + 255) / 256));
-  if (is_double)
-    hipLaunchKernelGGL((k_to_double<double>), gr, bl, 0, s, (const double*)a, b, n);
-  else
-    hipLaunchKernelGGL((k_to_double<float>), gr, bl, 0, s, (const float*)a, b, n);
-  return hipGetLastError();
-}
 hipError_t field_from_double(bool is_double, void* a, const double* b, size_t n, hipStream_t s) {
   if (n == 0) return hipSuccess;
   dim3 bl(256), gr(unsigned((n + 255) / 256));

@@ -23,7 +23,6 @@ hipError_t unpack_populations(int lattice, int storage, const void* f, double* o
                               const Geometry& g, int phase, hipStream_t s, int layout = LBM_LAYOUT_SOA);
 hipError_t pack_populations(int lattice, int storage, void* f, const double* in,
                             const Geometry& g, hipStream_t s, int layout = LBM_LAYOUT_SOA);
-hipError_t field_to_double(bool is_double, const void* a, double* b, size_t n, hipStream_t s);
 hipError_t field_from_double(bool is_double, void* a, const double* b, size_t n, hipStream_t s);
 
 }  // namespace lbmx

@@ -18,6 +18,7 @@
 
 #include "fields.hpp"
 #include "kernels.hpp"
+#include "readback.hpp"
 
 using namespace lbmx;
 
@@ -215,14 +216,22 @@ lbm_status put_field(lbm_ctx* c, void* field, const double* host, size_t count, 
   return LBM_OK;
 }
 
+// One field of `count` values (double, or float to be widened) into `host`.
+ReadBack field_read(bool is_double, const void* field, double* host, size_t count) {
+  if (is_double)
+    return {field, count * sizeof(double), sizeof(double),
+            [host](const char* data, size_t offset, size_t n) { std::memcpy((char*)host + offset, data, n); }};
+  return {field, count * sizeof(float), sizeof(float), [host](const char* data, size_t offset, size_t n) {
+            const float* a = reinterpret_cast<const float*>(data);
+            double* b = host + offset / sizeof(float);
+            for (size_t i = 0; i < n / sizeof(float); ++i) b[i] = double(a[i]);
+          }};
+}
+
 lbm_status get_field(lbm_ctx* c, const void* field, double* host, size_t count, int as = -1) {
-  double* tmp = nullptr;
   HIP_TRY(hipSetDevice(c->device));
-  HIP_TRY(hipMalloc(&tmp, count * sizeof(double)));
-  HIP_TRY(field_to_double(compute_double(as < 0 ? c->storage : as), field, tmp, count, c->stream));
-  HIP_TRY(hipMemcpyAsync(host, tmp, count * sizeof(double), hipMemcpyDeviceToHost, c->stream));
-  HIP_TRY(hipStreamSynchronize(c->stream));
-  HIP_TRY(hipFree(tmp));
+  const ReadBack r = field_read(compute_double(as < 0 ? c->storage : as), field, host, count);
+  HIP_TRY(read_back(c->device, c->stream, &r, 1));
   return LBM_OK;
 }
 
@@ -585,6 +594,7 @@ lbm_status lbm_ctx_create(lbm_ctx** out, int32_t lattice, int32_t storage,
   if (ndev < 1) return fail(LBM_ERR_NOT_FOUND, "no GPU visible");
   if (device < 0 || device >= ndev) return fail(LBM_ERR_INVALID_ARG, "device %d of %d", device, ndev);
   lbm_ctx* c = new lbm_ctx();
+  read_back_user(1);
   c->lattice = lattice;
   c->storage = storage;
   c->D = D;
@@ -650,6 +660,7 @@ lbm_status lbm_ctx_destroy(lbm_ctx* c) {
   if (c->ev1) (void)hipEventDestroy(c->ev1);
   if (c->stream) (void)hipStreamDestroy(c->stream);
   delete c;
+  read_back_user(-1);
   return LBM_OK;
 }
 
@@ -930,11 +941,14 @@ lbm_status lbm_init_equilibrium_field(lbm_ctx* c, const double* rho, const doubl
 
 lbm_status lbm_get_macros(lbm_ctx* c, double* rho, double* u) {
   if (!c) return fail(LBM_ERR_INVALID_ARG, "null ctx");
-  if (rho) {
-    lbm_status s = get_field(c, c->rho, rho, c->N);
-    if (s) return s;
-  }
-  if (u) return get_field(c, c->u, u, size_t(c->D) * c->N);
+  if (!rho && !u) return LBM_OK;
+  HIP_TRY(hipSetDevice(c->device));
+  const bool dbl = compute_double(c->storage);
+  ReadBack r[2];
+  int n = 0;
+  if (rho) r[n++] = field_read(dbl, c->rho, rho, c->N);
+  if (u) r[n++] = field_read(dbl, c->u, u, size_t(c->D) * c->N);
+  HIP_TRY(read_back(c->device, c->stream, r, n));
   return LBM_OK;
 }
 

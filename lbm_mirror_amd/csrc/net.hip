@@ -27,6 +27,7 @@
 #include <vector>
 
 #include "../../include/lbm_mirror_amd/lbm.h"
+#include "readback.hpp"
 
 namespace lbmnet {
 
@@ -1379,10 +1380,12 @@ lbm_status lbm_net_create(lbm_net** out, const lbm_net_config* cfg, int32_t devi
   lbm_net* n = new lbm_net();
   n->cfg = *cfg;
   n->device = device;
+  lbmx::read_back_user(1);
   lbm_status s = create_impl(n);
   if (s != LBM_OK) {
     free_all(n);
     delete n;
+    lbmx::read_back_user(-1);
     return s;
   }
   *out = n;
@@ -1395,6 +1398,7 @@ lbm_status lbm_net_destroy(lbm_net* n) {
   if (n->stream) (void)hipStreamSynchronize(n->stream);
   free_all(n);
   delete n;
+  lbmx::read_back_user(-1);
   return LBM_OK;
 }
 
@@ -1578,34 +1582,38 @@ lbm_status lbm_net_predict(lbm_net* n, uint32_t count, const uint8_t* flags, con
   if (!n || !flags || !u_max || !tau || !rho || !u) return nfail(LBM_ERR_INVALID_ARG, "null argument");
   NET_TRY(hipSetDevice(n->device));
   const size_t HW = size_t(n->cfg.height) * n->cfg.width;
-  std::vector<float> xf(size_t(n->cfg.batch) * HW * 8), yf(size_t(n->cfg.batch) * HW * 3);
+  std::vector<float> xf(size_t(n->cfg.batch) * HW * 8);
   NET_TRY(hipEventRecord(n->ev0, n->stream));
   for (uint32_t s = 0; s < count; s += n->cfg.batch) {
     const int B = int(std::min<uint32_t>(n->cfg.batch, count - s));
     for (int b = 0; b < B; ++b) host_features(n->cfg, flags + (s + b) * HW, u_max[s + b], tau[s + b], xf.data() + b * HW * 8);
     NS(upload_x(n, xf.data(), size_t(B) * HW * 8));
     NS(forward(n, B));
-    NET_TRY(hipMemcpyAsync(yf.data(), n->y, size_t(B) * HW * 3 * sizeof(float), hipMemcpyDeviceToHost, n->stream));
-    NET_TRY(hipStreamSynchronize(n->stream));
-    for (int b = 0; b < B; ++b) {
-      const size_t k = s + b;
-      const uint8_t* fl = flags + k * HW;
-      double* r = rho + k * HW;
-      double* ux = u + k * 2 * HW;
-      double* uy = ux + HW;
-      for (size_t i = 0; i < HW; ++i) {
-        const float* o = yf.data() + (b * HW + i) * 3;
-        if (fl[i] >= 2) {
-          ux[i] = (double(o[0]) * n->sd[0] + n->mu[0]) * u_max[k];
-          uy[i] = (double(o[1]) * n->sd[1] + n->mu[1]) * u_max[k];
-          r[i] = 1.0 + (double(o[2]) * n->sd[2] + n->mu[2]) * rho_unit(u_max[k]);
-        } else {
-          ux[i] = 0.0;
-          uy[i] = 0.0;
-          r[i] = 1.0;
+    auto denormalise = [&, s](const char* data, size_t offset, size_t bytes) {
+      const float* o = reinterpret_cast<const float*>(data);
+      const size_t p0 = offset / (3 * sizeof(float)), p1 = p0 + bytes / (3 * sizeof(float));
+      for (size_t p = p0; p < p1;) {  // image by image
+        const size_t k = s + p / HW, end = std::min(p1, (p / HW + 1) * HW);
+        const uint8_t* fl = flags + k * HW;
+        double* r = rho + k * HW;
+        double* ux = u + k * 2 * HW;
+        double* uy = ux + HW;
+        const double um = u_max[k], ru = rho_unit(um);
+        for (size_t i = p % HW; p < end; ++p, ++i, o += 3) {
+          if (fl[i] >= 2) {
+            ux[i] = (double(o[0]) * n->sd[0] + n->mu[0]) * um;
+            uy[i] = (double(o[1]) * n->sd[1] + n->mu[1]) * um;
+            r[i] = 1.0 + (double(o[2]) * n->sd[2] + n->mu[2]) * ru;
+          } else {
+            ux[i] = 0.0;
+            uy[i] = 0.0;
+            r[i] = 1.0;
+          }
         }
       }
-    }
+    };
+    const lbmx::ReadBack r{n->y, size_t(B) * HW * 3 * sizeof(float), 3 * sizeof(float), denormalise};
+    NET_TRY(lbmx::read_back(n->device, n->stream, &r, 1));
   }
   NET_TRY(hipEventRecord(n->ev1, n->stream));
   NET_TRY(hipEventSynchronize(n->ev1));
