@@ -889,6 +889,22 @@ __global__ void k_standardize(float* t, size_t n, float m0, float m1, float m2, 
 }
 
 // Minibatch assembly from the on-device training set.
+// Network input from the lattices' flags and the words of upload_features: 16
+// bytes a pixel.  (Laid out by the host this was 16 of the 20 ms of 16
+// predictions of 256 x 256.)
+__global__ void k_features(const uint8_t* flags, const uint32_t* tab, int B, int H, int W, uint16_t* x) {
+  const size_t i = size_t(blockIdx.x) * blockDim.x + threadIdx.x, HW = size_t(H) * W;
+  if (i >= B * HW) return;
+  const size_t b = i / HW;
+  const int r = int(i - b * HW), py = r / W, px = r - py * W;
+  const uint32_t* per = tab + H + W + b * (W + 1);
+  const uint32_t row = tab[py], col = tab[H + px], own = per[0], at = per[1 + px];
+  const uint32_t open = flags[i] >= 2 ? 0x3f80u : 0u;
+  // channels 0 .. 7: open, speed | tau, profile | x, y | pressure, blockage
+  reinterpret_cast<uint4*>(x)[i] =
+      make_uint4(open | (own << 16), (own >> 16) | (row << 16), (col & 0xffffu) | (row & 0xffff0000u), at);
+}
+
 __global__ void k_gather(const uint16_t* xs, const float* ts, const uint8_t* ms, const uint32_t* idx, int B, int HW,
                          uint16_t* x, float* t, uint8_t* m) {
   const size_t i = size_t(blockIdx.x) * blockDim.x + threadIdx.x;
@@ -959,6 +975,7 @@ struct lbm_net {
   uint16_t *ga[4] = {}, *gcat[3] = {}, *gpool[4] = {}, *gdec[3] = {}, *gbott = nullptr, *gy = nullptr;
   float *y = nullptr, *t = nullptr;
   uint8_t* msk = nullptr;
+  uint32_t* ftab = nullptr;  // upload_features' words
   float* partial = nullptr;
   size_t partial_n = 0;
   double* lpartial = nullptr;
@@ -1227,39 +1244,80 @@ lbm_status refresh_weights(lbm_net* n) {
 //   7 log((ny-2)/h(x)), the column's blockage.
 // Channels 6-7 carry the domain-wide resistance a 3x3-convolution stack
 // cannot integrate over its receptive field.
-void host_features(const lbm_net_config& cfg, const uint8_t* flags, double u_max, double tau, float* out) {
+// Channels 6 and 7 of a lattice's columns.
+void column_features(const lbm_net_config& cfg, const uint8_t* flags, double u_max, double tau, float* press,
+                     float* block) {
   const int H = cfg.height, W = cfg.width;
   const double nu = (tau - 0.5) / 3.0;
   double S = 0.0;  // inlet flux / u_max
   for (int y = 1; y < H - 1; ++y) S += 4.0 * (y - 0.5) * (H - 1.5 - y) / ((H - 2.0) * (H - 2.0));
-  std::vector<double> hcol(W), press(W);
-  for (int x = 0; x < W; ++x) {
-    int h = 0;
-    for (int y = 0; y < H; ++y) h += flags[size_t(y) * W + x] >= 2 ? 1 : 0;
-    hcol[x] = h > 0 ? double(h) : 1.0;
-  }
+  std::vector<int> h(W, 0);
+  for (int y = 0; y < H; ++y)
+    for (int x = 0; x < W; ++x) h[x] += flags[size_t(y) * W + x] >= 2 ? 1 : 0;
+  const double hfull = H > 2 ? double(H - 2) : 1.0;
   double acc = 0.0;
   for (int x = W - 1; x >= 0; --x) {
-    press[x] = 12.0 * nu * S * acc / u_max;
-    acc += 1.0 / (hcol[x] * hcol[x] * hcol[x]);
+    const double hcol = h[x] > 0 ? double(h[x]) : 1.0;
+    press[x] = float(std::log1p(12.0 * nu * S * acc / u_max));
+    block[x] = float(std::log(hfull / hcol));
+    acc += 1.0 / (hcol * hcol * hcol);
   }
-  const double hfull = H > 2 ? double(H - 2) : 1.0;
-  for (int y = 0; y < H; ++y) {
-    const double yy = y;
-    const double prof = 4.0 * (yy - 0.5) * (H - 1.5 - yy) / ((H - 2.0) * (H - 2.0));
+}
+float speed_feature(double u_max) { return float(u_max / 0.08); }
+float tau_feature(double tau) { return float((tau - 0.5) / 0.7); }
+float profile_feature(const lbm_net_config& cfg, int y) {
+  const double H = cfg.height, yy = y;
+  return float(4.0 * (yy - 0.5) * (H - 1.5 - yy) / ((H - 2.0) * (H - 2.0)));
+}
+float x_feature(const lbm_net_config& cfg, int x) { return float(double(x) / double(cfg.width - 1)); }
+float y_feature(const lbm_net_config& cfg, int y) { return float(double(y) / double(cfg.height - 1)); }
+
+void host_features(const lbm_net_config& cfg, const uint8_t* flags, double u_max, double tau, float* out) {
+  const int H = cfg.height, W = cfg.width;
+  std::vector<float> press(W), block(W);
+  column_features(cfg, flags, u_max, tau, press.data(), block.data());
+  for (int y = 0; y < H; ++y)
     for (int x = 0; x < W; ++x) {
       float* f = out + (size_t(y) * W + x) * 8;
-      const uint8_t fl = flags[size_t(y) * W + x];
-      f[0] = fl >= 2 ? 1.f : 0.f;
-      f[1] = float(u_max / 0.08);
-      f[2] = float((tau - 0.5) / 0.7);
-      f[3] = float(prof);
-      f[4] = float(double(x) / double(W - 1));
-      f[5] = float(double(y) / double(H - 1));
-      f[6] = float(std::log1p(press[x]));
-      f[7] = float(std::log(hfull / hcol[x]));
+      f[0] = flags[size_t(y) * W + x] >= 2 ? 1.f : 0.f;
+      f[1] = speed_feature(u_max);
+      f[2] = tau_feature(tau);
+      f[3] = profile_feature(cfg, y);
+      f[4] = x_feature(cfg, x);
+      f[5] = y_feature(cfg, y);
+      f[6] = press[x];
+      f[7] = block[x];
     }
+}
+
+// The network input of B lattices of `flags`, as bf16(host_features): the flags
+// and what the features depend on (row, column, lattice and its column, two
+// channels to a word) go to the device, where k_features lays them out.
+size_t feature_words(const lbm_net_config& cfg, int B) {
+  return size_t(cfg.height) + cfg.width + size_t(B) * (cfg.width + 1);
+}
+lbm_status upload_features(lbm_net* n, int B, const uint8_t* flags, const double* u_max, const double* tau,
+                           std::vector<uint32_t>& tab) {
+  const int H = n->cfg.height, W = n->cfg.width;
+  const size_t HW = size_t(H) * W;
+  auto two = [](float lo, float hi) { return uint32_t(f2bf(lo)) | (uint32_t(f2bf(hi)) << 16); };
+  tab.resize(feature_words(n->cfg, B));
+  uint32_t* rows = tab.data();
+  uint32_t* cols = rows + H;
+  uint32_t* per = cols + W;
+  for (int y = 0; y < H; ++y) rows[y] = two(profile_feature(n->cfg, y), y_feature(n->cfg, y));
+  for (int x = 0; x < W; ++x) cols[x] = two(x_feature(n->cfg, x), 0.f);
+  std::vector<float> press(W), block(W);
+  for (int b = 0; b < B; ++b, per += W + 1) {
+    column_features(n->cfg, flags + b * HW, u_max[b], tau[b], press.data(), block.data());
+    per[0] = two(speed_feature(u_max[b]), tau_feature(tau[b]));
+    for (int x = 0; x < W; ++x) per[1 + x] = two(press[x], block[x]);
   }
+  NET_TRY(hipMemcpyAsync(n->msk, flags, B * HW, hipMemcpyHostToDevice, n->stream));
+  NET_TRY(hipMemcpyAsync(n->ftab, tab.data(), tab.size() * sizeof(uint32_t), hipMemcpyHostToDevice, n->stream));
+  hipLaunchKernelGGL(k_features, dim3(blocks_for(B * HW)), dim3(256), 0, n->stream, n->msk, n->ftab, B, H, W, n->x);
+  NET_TRY(hipGetLastError());
+  return LBM_OK;
 }
 
 lbm_status upload_x(lbm_net* n, const float* x, size_t count) {
@@ -1275,7 +1333,7 @@ void free_all(lbm_net* n) {
     (void)hipFree(L.wb);
     (void)hipFree(L.wt);
   }
-  void* ps[] = {n->w,        n->g,     n->m1,      n->m2,   n->y,  n->t,  n->msk, n->partial,
+  void* ps[] = {n->w,        n->g,     n->m1,      n->m2,   n->y,  n->t,  n->msk, n->ftab, n->partial,
                 n->lpartial, n->dloss, n->dlosses, n->didx, n->xs, n->ts, n->ms};
   for (void* p : ps) (void)hipFree(p);
   for (uint16_t* p : {n->x, n->bott, n->gbott, n->gy}) afree(p);
@@ -1327,6 +1385,7 @@ lbm_status create_impl(lbm_net* n) {
   NS(dalloc(&n->y, level_pixels(n, 0) * 3));
   NS(dalloc(&n->t, level_pixels(n, 0) * 3));
   NS(dalloc(&n->msk, level_pixels(n, 0)));
+  NS(dalloc(&n->ftab, feature_words(n->cfg, c.batch)));
   size_t pmax = 0;
   for (const Layer& L : n->layers) {
     int splits, chunk;
@@ -1582,13 +1641,16 @@ lbm_status lbm_net_predict(lbm_net* n, uint32_t count, const uint8_t* flags, con
   if (!n || !flags || !u_max || !tau || !rho || !u) return nfail(LBM_ERR_INVALID_ARG, "null argument");
   NET_TRY(hipSetDevice(n->device));
   const size_t HW = size_t(n->cfg.height) * n->cfg.width;
-  std::vector<float> xf(size_t(n->cfg.batch) * HW * 8);
+  std::vector<uint32_t> tab;
   NET_TRY(hipEventRecord(n->ev0, n->stream));
   for (uint32_t s = 0; s < count; s += n->cfg.batch) {
     const int B = int(std::min<uint32_t>(n->cfg.batch, count - s));
-    for (int b = 0; b < B; ++b) host_features(n->cfg, flags + (s + b) * HW, u_max[s + b], tau[s + b], xf.data() + b * HW * 8);
-    NS(upload_x(n, xf.data(), size_t(B) * HW * 8));
-    NS(forward(n, B));
+    lbm_status st = upload_features(n, B, flags + s * HW, u_max + s, tau + s, tab);
+    if (st == LBM_OK) st = forward(n, B);
+    if (st != LBM_OK) {
+      (void)hipStreamSynchronize(n->stream);  // `tab` may still be read
+      return st;
+    }
     auto denormalise = [&, s](const char* data, size_t offset, size_t bytes) {
       const float* o = reinterpret_cast<const float*>(data);
       const size_t p0 = offset / (3 * sizeof(float)), p1 = p0 + bytes / (3 * sizeof(float));
