@@ -632,11 +632,24 @@ lbm_status lbm_ctx_create(lbm_ctx** out, int32_t lattice, int32_t storage,
   if (e != hipSuccess)
     return bail(fail(e == hipErrorOutOfMemory ? LBM_ERR_OUT_OF_MEMORY : LBM_ERR_CRITICAL,
                      "allocation: %s", hipGetErrorString(e)));
-  // block shape: one row segment of up to 256 cells, rows stacked to fill 256 threads
+  // Block shape: one row segment of up to 256 cells, rows stacked to fill 256
+  // threads; 128 cells where blocks of 256 would leave over a third of their
+  // lanes without a cell (rows of 257 to 341 cells; us per step at 300 x 100 x 60:
+  // D3Q19 F32 73 for 84, F64 115 for 149, F16 40 for 46, D3Q27 F32 103 for 118;
+  // at 400 and 520 cells 256 are as fast or faster).  D3Q27 FP64 has one or two
+  // wavefronts per SIMD, and takes one-row blocks of 64 or 128 cells, whichever
+  // leaves fewer lanes idle, which end sooner: 128 x 100 x 60 52 us for 66, 64^3 21
+  // for 28, 256 x 128 x 64 177 for 181.
   int bx = 64;
   while (bx < 256 && uint64_t(bx) < n[0]) bx *= 2;
+  auto lanes = [&](uint64_t w) { return (n[0] + w - 1) / w * w; };
+  if (bx == 256 && (lanes(256) - n[0]) * 3 > lanes(256) && n[0] > 256) bx = 128;
   c->shape.bx = bx;
   c->shape.by = 256 / bx;
+  if (lattice == LBM_D3Q27 && storage == LBM_F64) {
+    c->shape.bx = lanes(64) < lanes(128) ? 64 : 128;
+    c->shape.by = 1;
+  }
   // step graphs pay off where launches are a visible share of a step; past
   // 2^20 cells (a 200 µs step at 8 M cells) they change nothing but cost a
   // capture

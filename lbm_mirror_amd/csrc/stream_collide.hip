@@ -87,11 +87,12 @@ __device__ __forceinline__ void st_even(P p, T v, T w) {
 #ifndef LBMX_BUF_Q27
 #define LBMX_BUF_Q27 3
 #endif
-// FP32 storage only: where it was measured (the D2Q9 FP64 step, C1, is 2%
-// slower in the buffer form)
+// FP64: D3Q27 alone (the D2Q9 FP64 step, C1, is 2% slower in the buffer form);
+// 16-bit storage on every lattice, in both phases (the figures at launch_t).
 template <class L, class S>
 constexpr int buf_phases() {
-  if (sizeof(S) != 4) return 0;
+  if (sizeof(S) == 2) return 3;
+  if (sizeof(S) == 8) return L::Q == 27 ? 3 : 0;
   return L::Q == 9 ? LBMX_BUF_Q9 : (L::Q == 19 ? LBMX_BUF_Q19 : LBMX_BUF_Q27);
 }
 // AUX: cache policy of the access (2: nontemporal)
@@ -173,20 +174,34 @@ constexpr int aux_odd_st() { return (sizeof(S) == 4 && sizeof(T) == 4 && (LBMX_N
 #ifndef LBMX_WAVES_Q9
 #define LBMX_WAVES_Q9 8
 #endif
-template <class L, class T, bool ODD, bool BUF>
+template <class L, class T, bool ODD, bool BUF, bool ROW1>
 struct StepWaves {
   static constexpr int value = 1;
 };
+// FP64: D3Q19 takes 184 to 222 registers, two wavefronts per SIMD; held to three,
+// blocks of several rows (the narrower lattices) run 9% faster (97 x 61 x 45 19.7 ->
+// 18.0 us, 64^3 16.7 -> 15.2), one-row blocks 1% slower (256 x 128 x 128 232 -> 234
+// us), and four spill (350 us).  D3Q27 in the buffer form takes all 256 and one
+// wavefront; held to two: 128 x 100 x 60 58 -> 52 us, 64^3 28 -> 22 us, 256 x 128 x
+// 64 180 -> 177 us (three spill, 271 us).
 template <bool ODD, bool BUF>
-struct StepWaves<D3Q19, float, ODD, BUF> {
+struct StepWaves<D3Q19, double, ODD, BUF, false> {
+  static constexpr int value = 3;
+};
+template <bool ODD>
+struct StepWaves<D3Q27, double, ODD, true, false> {
+  static constexpr int value = 2;
+};
+template <bool ODD, bool BUF, bool ROW1>
+struct StepWaves<D3Q19, float, ODD, BUF, ROW1> {
   static constexpr int value = LBMX_WAVES_Q19;
 };
-template <bool ODD, bool BUF>
-struct StepWaves<D3Q27, float, ODD, BUF> {
+template <bool ODD, bool BUF, bool ROW1>
+struct StepWaves<D3Q27, float, ODD, BUF, ROW1> {
   static constexpr int value = (ODD || !BUF) ? LBMX_WAVES_Q27_ODD : LBMX_WAVES_Q27;
 };
-template <bool ODD, bool BUF>
-struct StepWaves<D2Q9, float, ODD, BUF> {
+template <bool ODD, bool BUF, bool ROW1>
+struct StepWaves<D2Q9, float, ODD, BUF, ROW1> {
   static constexpr int value = LBMX_WAVES_Q9;
 };
 // ROW1: every block is one row segment (blockDim.y == 1), so y and z, the
@@ -194,7 +209,7 @@ struct StepWaves<D2Q9, float, ODD, BUF> {
 // (scalar registers) and each population access is a uniform row base plus
 // a 32-bit per-lane x offset; only x and its two neighbours live per lane.
 template <class L, class S, class T, bool WB, bool ODD, bool BUF, bool ROW1>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(StepWaves<L, T, ODD, BUF>::value))) void k_aa_step(
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(StepWaves<L, T, ODD, BUF, ROW1>::value))) void k_aa_step(
     StepArgs a) {
   constexpr int Q = L::Q;
   const int x = blockIdx.x * blockDim.x + threadIdx.x;
@@ -389,7 +404,9 @@ __global__ __launch_bounds__(1024) void k_aa_row(StepArgs a) {
 // mode).  Phase-1 loads are all issued before any value is used (no load in
 // a per-lane branch); where a pair would cross the row's end (periodic wrap,
 // or the zero ghost ring) the word is clamped into the row and the missing
-// value loaded on its own, and such pairs are stored one value at a time.
+// value loaded on its own, and such pairs are stored one value at a time; only
+// the wavefronts that hold a row end, or lie in a row without all neighbour
+// rows, spend instructions on either.
 // Even rows only (nx even); every element is still read and written by
 // exactly one thread.
 template <class S>
@@ -408,8 +425,12 @@ struct Bits16<__hip_bfloat16> {
 #ifndef LBMX_NT_PAIR
 #define LBMX_NT_PAIR 3
 #endif
+// D3Q19 F16 at 512 x 128 x 128: phase 0 117 us, phase 1 187 us with the row
+// ends decided per lane and direction (845 vector instructions a cell for 617),
+// about 150 us with them decided per wavefront; held to 4 wavefronts per SIMD
+// (phase 0 took 150 registers) both phases gain another 3%; 5 spill (x 1.7).
 template <class L, class S, bool ODD>
-__global__ __launch_bounds__(256) void k_aa_pair(StepArgs a) {
+__global__ __launch_bounds__(256, 4) void k_aa_pair(StepArgs a) {
   using T = float;
   constexpr int Q = L::Q;
   using G16 = __attribute__((address_space(1))) uint16_t;
@@ -431,8 +452,11 @@ __global__ __launch_bounds__(256) void k_aa_pair(StepArgs a) {
                          uint32_t(z == nz - 1 ? 0 : z + 1) * sxy};
   const bool VY[3] = {y > 0 || py, true, y < ny - 1 || py};
   const bool VZ[3] = {L::D < 3 || z > 0 || pz, true, L::D < 3 || z < nz - 1 || pz};
-  // the x position of x + d inside the row, or -1 in the ghost ring
-  auto wrap = [&](int x) -> int { return x < 0 ? (px ? x + nx : -1) : (x >= nx ? (px ? x - nx : -1) : x); };
+  // What is no more than this for most wavefronts, decided for a whole one: its
+  // neighbour rows exist, and it holds no row end.
+  const bool inner = VY[0] && VY[2] && VZ[0] && VZ[2];
+  const bool first = x0 == 0, last = x0 == nx - 2;
+  const bool ends = __any(first || last);
 
   T f[2][Q];
   if (!ODD) {
@@ -460,11 +484,8 @@ __global__ __launch_bounds__(256) void k_aa_pair(StepArgs a) {
       const int xa = L::cx[i] > 0 ? (xs < 0 ? 0 : xs) : (L::cx[i] < 0 ? (xs > nx - 2 ? nx - 2 : xs) : xs);
       raw[i] = *(const G32u*)(fb + (size_t(L::opp[i]) * Np + rb + uint32_t(xa)));
     }
-    const bool first = x0 == 0, last = x0 == nx - 2;
-    uint32_t edge[Q];
-#pragma unroll
-    for (int i = 0; i < Q; ++i) edge[i] = 0u;
-    if (__any(first || last)) {  // the wavefronts that hold a row end
+    if (ends) {  // the wavefronts that hold a row end
+      uint32_t edge[Q];
 #pragma unroll
       for (int i = 0; i < Q; ++i) {
         if (L::cx[i] == 0) continue;
@@ -472,25 +493,29 @@ __global__ __launch_bounds__(256) void k_aa_pair(StepArgs a) {
         const uint32_t rb = (VY[iy] && VZ[iz]) ? Y[iy] + Z[iz] : row;
         edge[i] = fb[size_t(L::opp[i]) * Np + rb + uint32_t(L::cx[i] > 0 ? nx - 1 : 0)];
       }
+#pragma unroll
+      for (int i = 0; i < Q; ++i) {
+        if (L::cx[i] > 0) raw[i] = first ? (edge[i] | (raw[i] << 16)) : raw[i];
+        if (L::cx[i] < 0) raw[i] = last ? ((raw[i] >> 16) | (edge[i] << 16)) : raw[i];
+      }
     }
 #pragma unroll
     for (int i = 0; i < Q; ++i) {
-      const int iy = 1 - L::cy[i], iz = 1 - L::cz[i];
-      const bool rv = VY[iy] && VZ[iz];
-      uint32_t lo = raw[i] & 0xffffu, hi = raw[i] >> 16;
-      bool g0 = !rv, g1 = !rv;
-      if (L::cx[i] > 0) {
-        hi = first ? lo : hi;
-        lo = first ? edge[i] : lo;
-        g0 = g0 || (first && !px);
-      } else if (L::cx[i] < 0) {
-        lo = last ? hi : lo;
-        hi = last ? edge[i] : hi;
-        g1 = g1 || (last && !px);
-      }
       const T w = T(L::w[i]);
-      f[0][i] = g0 ? T(0) : Bits16<S>::f(lo) + w;
-      f[1][i] = g1 ? T(0) : Bits16<S>::f(hi) + w;
+      f[0][i] = Bits16<S>::f(raw[i] & 0xffffu) + w;
+      f[1][i] = Bits16<S>::f(raw[i] >> 16) + w;
+    }
+    if (ends && !px) {  // the ghost ring's zeros at the row's ends
+#pragma unroll
+      for (int i = 0; i < Q; ++i) {
+        if (L::cx[i] > 0) f[0][i] = first ? T(0) : f[0][i];
+        if (L::cx[i] < 0) f[1][i] = last ? T(0) : f[1][i];
+      }
+    }
+    if (!inner) {  // and in its rows
+#pragma unroll
+      for (int i = 0; i < Q; ++i)
+        if (!(VY[1 - L::cy[i]] && VZ[1 - L::cz[i]])) f[0][i] = f[1][i] = T(0);
     }
   }
 
@@ -508,32 +533,48 @@ __global__ __launch_bounds__(256) void k_aa_pair(StepArgs a) {
       else *p = v;
     }
   } else {
+    uint32_t v[Q];
 #pragma unroll
     for (int i = 0; i < Q; ++i) {
       const T w = T(L::w[i]);
-      const uint32_t b0 = Bits16<S>::b(f[0][i] - w), b1 = Bits16<S>::b(f[1][i] - w);
+      v[i] = Bits16<S>::b(f[0][i] - w) | (Bits16<S>::b(f[1][i] - w) << 16);
+    }
+    // the words whose two destinations lie in one row
+#pragma unroll
+    for (int i = 0; i < Q; ++i) {
       const int jy = 1 + L::cy[i], jz = 1 + L::cz[i];
-      const int xd = x0 + L::cx[i];  // the destination of cell x0 (x0 + 1's is xd + 1)
-      if (VY[jy] && VZ[jz]) {
+      if (!inner && !(VY[jy] && VZ[jz])) continue;
+      G32u* p = (G32u*)(fb + (size_t(i) * Np + Y[jy] + Z[jz]) + uint32_t(x0 + L::cx[i]));
+      if (L::cx[i] == 0 || !ends) *p = v[i];
+      else if (L::cx[i] > 0 ? !last : !first) *p = v[i];
+    }
+    if (first || last) {  // the others, one value at a time
+#pragma unroll
+      for (int i = 0; i < Q; ++i) {
+        if (L::cx[i] == 0) continue;
+        const int jy = 1 + L::cy[i], jz = 1 + L::cz[i];
+        if (!(VY[jy] && VZ[jz])) continue;
         G16* base = fb + (size_t(i) * Np + Y[jy] + Z[jz]);
-        if (xd >= 0 && xd + 1 < nx) {
-          *(G32u*)(base + uint32_t(xd)) = b0 | (b1 << 16);
-        } else {
-          const int d0 = wrap(xd), d1 = wrap(xd + 1);
-          if (d0 >= 0) base[d0] = (uint16_t)b0;
-          if (d1 >= 0) base[d1] = (uint16_t)b1;
+        if (L::cx[i] > 0 && last) {
+          base[nx - 1] = uint16_t(v[i]);
+          if (px) base[0] = uint16_t(v[i] >> 16);
+        }
+        if (L::cx[i] < 0 && first) {
+          base[0] = uint16_t(v[i] >> 16);
+          if (px) base[nx - 1] = uint16_t(v[i]);
         }
       }
-      // a cell whose upstream neighbour is in the ghost ring: its own slot
-      // takes the ghost's zero (nobody else streams into it)
-      const int uy = 1 - L::cy[i], uz = 1 - L::cz[i];
-      const bool rows_ok = VY[uy] && VZ[uz];
-      const bool up0 = rows_ok && wrap(x0 - L::cx[i]) >= 0, up1 = rows_ok && wrap(x0 + 1 - L::cx[i]) >= 0;
-      if (!up0 || !up1) {
+    }
+    // a cell whose upstream neighbour is in the ghost ring: its own slot
+    // takes the ghost's zero (nobody else streams into it)
+    if (!inner || (ends && !px)) {
+#pragma unroll
+      for (int i = 0; i < Q; ++i) {
+        const bool rows_ok = VY[1 - L::cy[i]] && VZ[1 - L::cz[i]];
         G16* own = fb + (size_t(i) * Np + row + uint32_t(x0));
-        const uint32_t zb = Bits16<S>::b(T(0) - w);
-        if (!up0) own[0] = (uint16_t)zb;
-        if (!up1) own[1] = (uint16_t)zb;
+        const uint16_t zb = uint16_t(Bits16<S>::b(T(0) - T(L::w[i])));
+        if (!rows_ok || (L::cx[i] > 0 && first && !px)) own[0] = zb;
+        if (!rows_ok || (L::cx[i] < 0 && last && !px)) own[1] = zb;
       }
     }
   }
@@ -901,12 +942,20 @@ hipError_t launch_batch_residual(int dims, int storage, const BatchArgs& b, cons
 
 template <class L, class S, class T, bool WB>
 static hipError_t launch_t(bool odd, const StepArgs& a, const LaunchShape& sh, hipStream_t s) {
-  // 16-bit storage, even rows: two cells per thread (form 3; the default for
-  // D2Q9 and D3Q19, D3Q27's 54 values per thread spill); one-row blocks of
-  // sh.bx threads over the row's pairs
+  // 16-bit storage.  Populations that stay in the 256 MiB last-level cache: one
+  // cell per thread through the buffer resource (D3Q19 F16, us per step, against
+  // two cells per thread: 64^3 7.7 / 12.6, 200 x 80 x 60 22.7 / 27.2,
+  // 400 x 128 x 128 119 / 136; D2Q9 1024 x 512 6.8 / 9.0): more wavefronts to
+  // hide the cache's latency.  Beyond it even rows take two cells per thread
+  // (form 3), FP32's bytes per memory instruction: D3Q19 512 x 128 x 128 131 /
+  // 146, D2Q9 4096 x 4096 119 / 131; not D3Q27, whose 54 values spill (512 x
+  // 128 x 128 buffer resource 236, global addresses 258).
+  constexpr uint64_t kLastLevel = uint64_t(256) << 20;
+  const uint64_t bytes = uint64_t(L::Q) * a.Np * sizeof(S);
   if constexpr (sizeof(S) == 2) {
     const int form = sh.form[odd ? 1 : 0];
-    if ((form == 3 || (form == 0 && L::Q <= 19)) && a.nx % 2 == 0) {
+    if ((form == 3 || (form == 0 && L::Q <= 19 && bytes > kLastLevel)) && a.nx % 2 == 0) {
+      // one-row blocks of sh.bx threads over the row's pairs
       const int pairs = a.nx / 2;
       int bx = 64;
       while (bx < pairs && bx < sh.bx) bx *= 2;
@@ -936,7 +985,7 @@ static hipError_t launch_t(bool odd, const StepArgs& a, const LaunchShape& sh, h
   // the buffer-resource form where the population array's bytes fit the 32-bit range
   const int form = sh.form[odd ? 1 : 0];
   const bool want_buf = form == 0 ? (buf_phases<L, S>() & (odd ? 2 : 1)) != 0 : form == 2;
-  const bool buf = want_buf && uint64_t(L::Q) * a.Np * sizeof(S) <= 0xffffffffull;
+  const bool buf = want_buf && bytes <= 0xffffffffull;
   // one-row blocks take the row-uniform addressing in the global form
   // (D3Q19 FP32 1%, D2Q9 FP64 10% faster); the buffer form keeps per-lane
   // rows (row-uniform scalar offsets are 4% slower in D3Q27 phase 1, 3% in
