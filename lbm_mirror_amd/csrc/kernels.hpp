@@ -132,6 +132,7 @@ hipError_t launch_segment_sums(const double* partial, const uint32_t* begin, uin
                                hipStream_t s);
 
 // Particle coupling (particles.hip)
+constexpr int kBoxInts = 18;
 struct ParticleArgs {
   // lattice and fields
   const void* f;
@@ -178,11 +179,11 @@ struct ParticleArgs {
   int32_t fixed_axis;  // ParticleAxisIntegrate instead of ParticleIntegrate
   double axis[3];      // its normalised axis, T-rounded (2D: the sign in [0])
   uint32_t* status;    // the context's fault words (StepArgs::status)
-  // PSM scatter porosity without the per-cell reset: n*12 ints, particle p's
-  // box of this gather at [12p, 12p+6) (lo, hi) and of the previous one at
-  // [12p+6, 12p+12).  The gather sweeps the union of the two and sets the
-  // cells of the previous box that no current box holds back to 1 (null:
-  // every cell is reset before the gather)
+  // PSM and HLBM scatter porosity without the per-cell reset: kBoxInts ints per
+  // particle, its box (lo, hi) of this gather, of the previous one, and of the
+  // last HLBM stamp.  The gather sweeps the union of the three, sets the cells
+  // of the previous box that no current box holds back to 1, and the stamped
+  // cells' N and D back to 0 (null: every cell is reset before the gather)
   int32_t* boxes;
 };
 
@@ -200,7 +201,8 @@ enum PartField {
 hipError_t launch_psm_couple(int lattice, int storage, const ParticleArgs& a, hipStream_t s);
 // Porosity 1 in every cell and every particle's previous box empty: the
 // state from which the gathers keep the porosity without a per-cell reset
-hipError_t launch_sweep_reset(bool dbl, void* por, uint32_t N, int32_t* boxes, uint32_t n, hipStream_t s);
+hipError_t launch_sweep_reset(bool dbl, int dims, void* por, void* pn, void* pd, uint32_t N, int32_t* boxes, uint32_t n,
+                              hipStream_t s);
 // HLBM stamp after the move: N += u_p (1 - B), D += 1 - B over each post-move AABB
 hipError_t launch_hlbm_stamp(int dims, int storage, const ParticleArgs& a, hipStream_t s);
 hipError_t launch_dem_contact(int dims, int storage, const ParticleArgs& a, hipStream_t s);

@@ -132,8 +132,8 @@ struct lbm_ctx {
   uint64_t* cl_slot = nullptr;
   uint64_t* cl_overflow = nullptr;
   uint32_t* owner = nullptr;
-  // PSM scatter porosity kept by the gathers' sweeps (ParticleArgs::boxes):
-  // 12 ints per particle; por_fresh once the porosity is 1 outside the
+  // scatter porosity kept by the gathers' sweeps (ParticleArgs::boxes):
+  // kBoxInts ints per particle; por_fresh once the porosity is 1 outside the
   // previous boxes (after a full reset, kept by every sweep since)
   int32_t* boxes = nullptr;
   bool por_fresh = false;
@@ -269,10 +269,10 @@ void spin_axis_normalised(int D, const double* in, double* out) {
 #endif
 constexpr uint64_t kGatherCells = LBMX_GATHER_CELLS;
 
-// PSM coupling with scatter porosity and per-block ownership: the gathers
-// keep the porosity without a per-cell reset
+// PSM or HLBM coupling with scatter porosity and per-block ownership: the
+// gathers keep the porosity (and HLBM's N and D) without a per-cell reset
 bool sweep_eligible(const lbm_ctx* c) {
-  return c->np > 0 && c->boxes && c->pp.coupling == LBM_COUPLING_PSM &&
+  return c->np > 0 && c->boxes && c->pp.coupling != LBM_COUPLING_FPLBM &&
          c->pp.porosity_mode == LBM_POROSITY_SCATTER && !c->owner;
 }
 bool sweep_ready(const lbm_ctx* c) { return sweep_eligible(c) && c->por_fresh; }
@@ -281,7 +281,9 @@ bool sweep_ready(const lbm_ctx* c) { return sweep_eligible(c) && c->por_fresh; }
 // boxes) where the porosity was set from outside or the particles changed
 lbm_status prepare_sweep(lbm_ctx* c) {
   if (!sweep_eligible(c) || c->por_fresh) return LBM_OK;
-  HIP_TRY(launch_sweep_reset(c->storage == LBM_F64, c->por, c->N, c->boxes, c->np, c->stream));
+  const bool hlbm = c->pp.coupling == LBM_COUPLING_HLBM;
+  HIP_TRY(launch_sweep_reset(c->storage == LBM_F64, c->D, c->por, hlbm ? c->pn : nullptr, hlbm ? c->pd : nullptr, c->N,
+                             c->boxes, c->np, c->stream));
   c->por_fresh = true;
   return LBM_OK;
 }
@@ -1320,7 +1322,7 @@ lbm_status lbm_particles_set(lbm_ctx* c, const lbm_particle* p, uint32_t n,
     c->boxes = nullptr;
     c->np = 0;
     if (n > 0) {
-      HIP_TRY(alloc_zero((void**)&c->boxes, size_t(n) * 12 * sizeof(int32_t), c->stream));
+      HIP_TRY(alloc_zero((void**)&c->boxes, size_t(n) * kBoxInts * sizeof(int32_t), c->stream));
       HIP_TRY(alloc_zero(&c->parts, size_t(n) * kPartFields * (dbl ? 8 : 4), c->stream));
       HIP_TRY(alloc_zero(&c->snap, size_t(n) * kPartFields * (dbl ? 8 : 4), c->stream));
       HIP_TRY(alloc_zero((void**)&c->f64, size_t(n) * 3 * sizeof(double), c->stream));

@@ -86,6 +86,101 @@ __device__ __forceinline__ T pop_sel(const ParticleArgs& a, int i, int x, int y,
   return ok ? v : T(0);
 }
 
+// f_i at x and f_opp(i) at x + c_i for every direction (pop_sel of both).  What
+// lies 1 and 2 cells away along each axis is worked out once; a direction then
+// adds three offsets, always to a cell of the lattice (where its own lies
+// outside, the axis keeps x), and its validity is a mask of one word's bits,
+// looked at when every load has been issued.  With a select per load the phase-1
+// gather waited for most of its loads one by one: a single D3Q27 sphere 12 us in
+// phase 0 and 19 us in phase 1, 9 and 10 us now; 200 discs 10.4 and 13.3, 10 us now
+// in both.
+template <int BYTES>
+struct RawBits;
+template <>
+struct RawBits<2> {
+  using type = uint16_t;
+};
+template <>
+struct RawBits<4> {
+  using type = uint32_t;
+};
+template <>
+struct RawBits<8> {
+  using type = uint64_t;
+};
+template <class L, class S, class T>
+__device__ __forceinline__ void gather_pops(const ParticleArgs& a, const int (&x)[3], T (&fi)[L::Q], T (&fo)[L::Q]) {
+  using Raw = typename RawBits<sizeof(S)>::type;
+  using G = const __attribute__((address_space(1))) Raw;
+  G* f = (G*)a.f;
+  const int n[3] = {a.nx, a.ny, a.nz};
+  const uint32_t stride[3] = {1u, uint32_t(a.nx), uint32_t(a.nx) * uint32_t(a.ny)};
+  uint32_t at[3][5];  // the axis' part of the cell index at offsets -2 .. 2
+  uint32_t out = 0;   // bit 5 d + 2 + o: offset o along d lies outside
+#pragma unroll
+  for (int d = 0; d < L::D; ++d) {
+    const bool per = a.periodic & (1u << d);
+    at[d][2] = uint32_t(x[d]) * stride[d];
+#pragma unroll
+    for (int side = -1; side <= 1; side += 2) {
+      int v = x[d];
+      bool ok = true;
+#pragma unroll
+      for (int k = 1; k <= 2; ++k) {
+        v += side;
+        if (v < 0 || v >= n[d]) {
+          ok = ok && per;
+          v = side < 0 ? n[d] - 1 : 0;
+        }
+        at[d][2 + side * k] = uint32_t(ok ? v : x[d]) * stride[d];
+        out |= ok ? 0u : 1u << (5 * d + 2 + side * k);
+      }
+    }
+  }
+  auto cell = [&](int i, int times) {  // x + times * c_i
+    uint32_t c = 0;
+#pragma unroll
+    for (int d = 0; d < L::D; ++d) c += at[d][2 + times * cdir<L>(i, d)];
+    return c;
+  };
+  auto value = [&](Raw raw, int i, int times) {
+    uint32_t mask = 0;
+#pragma unroll
+    for (int d = 0; d < L::D; ++d)
+      if (times * cdir<L>(i, d) != 0) mask |= 1u << (5 * d + 2 + times * cdir<L>(i, d));
+    S own;
+    __builtin_memcpy(&own, &raw, sizeof own);
+    const T v = ldp<S, T>(&own, T(L::w[i]));
+    return (out & mask) ? T(0) : v;
+  };
+  Raw ri[L::Q], ro[L::Q];
+  if (a.phase == 0) {
+#pragma unroll
+    for (int i = 1; i < L::Q; ++i) {
+      ri[i] = f[size_t(i) * a.Np + cell(i, 0)];
+      ro[i] = f[size_t(L::opp[i]) * a.Np + cell(i, 1)];
+    }
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int i = 1; i < L::Q; ++i) {
+      fi[i] = value(ri[i], i, 0);
+      fo[i] = value(ro[i], i, 1);
+    }
+  } else {
+#pragma unroll
+    for (int i = 1; i < L::Q; ++i) {
+      ri[i] = f[size_t(L::opp[i]) * a.Np + cell(i, -1)];
+      ro[i] = f[size_t(i) * a.Np + cell(i, 2)];
+    }
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int i = 1; i < L::Q; ++i) {
+      fi[i] = value(ri[i], i, -1);
+      fo[i] = value(ro[i], i, 2);
+    }
+  }
+}
+
 template <class T, int D>
 struct Box {
   int lo[3], hi[3];
@@ -199,6 +294,13 @@ __global__ __launch_bounds__(256) void k_hlbm_stamp(ParticleArgs a) {
   const T* parts = static_cast<const T*>(a.parts);
   const T* P = parts + size_t(p) * kPartFields;
   const Box<T, D> b = aabb_of<T, D>(P, a);
+  if (a.boxes && chunk == 0 && threadIdx.x == 0) {  // for the next gather's sweep
+#pragma unroll
+    for (int d = 0; d < 3; ++d) {
+      a.boxes[size_t(p) * kBoxInts + 12 + d] = b.lo[d];
+      a.boxes[size_t(p) * kBoxInts + 15 + d] = b.hi[d];
+    }
+  }
   const T ts = T(1.0) / T(a.sub_steps == 0 ? uint64_t(1) : a.sub_steps);
   T vp[3] = {T(0), T(0), T(0)};
   stamp_velocity<T, D>(P, ts, vp);
@@ -461,54 +563,86 @@ __global__ __launch_bounds__(256) void k_gather(ParticleArgs a) {
   __shared__ uint32_t lo_q[kOverlapCap];
   __shared__ int lo_box[kOverlapCap][6];
   const LocalOwners<T, D> lo{&lo_cnt, lo_q, lo_box};
-  // the sweep (PSM scatter porosity without the per-cell reset): the cells of
-  // this gather's box and of the previous gather's box, whose cells outside
-  // every current box go back to porosity 1
-  constexpr bool kCanSweep = CPL == kCplPsm && LOCAL;
+  // the sweep (scatter porosity without the per-cell reset): the cells of this
+  // gather's box and of the previous gather's box, whose cells outside every
+  // current box go back to porosity 1; HLBM, the cells of the last stamp's box
+  // too, whose N and D go back to 0
+  constexpr bool kCanSweep = !fplbm && LOCAL;
   const bool sweep = kCanSweep && a.boxes != nullptr && scatter;
-  Box<T, D> bp, R = b;
+  Box<T, D> bp, bs, R = b;
   if (kCanSweep && sweep) {
-    const int32_t* pb = a.boxes + size_t(p) * 12 + 6;
-    bp.count = 1;
-    for (int d = 0; d < 3; ++d) {
-      bp.lo[d] = pb[d];
-      bp.hi[d] = pb[3 + d];
-      bp.count *= uint32_t(bp.hi[d] - bp.lo[d]);
-    }
-    if (b.count == 0) {
-      R = bp;
-    } else if (bp.count > 0) {
-      R.count = 1;
+    const int32_t* pb = a.boxes + size_t(p) * kBoxInts;
+    auto read = [&](int at) {
+      Box<T, D> o;
+      o.count = 1;
+#pragma unroll
       for (int d = 0; d < 3; ++d) {
-        R.lo[d] = min(b.lo[d], bp.lo[d]);
-        R.hi[d] = max(b.hi[d], bp.hi[d]);
+        o.lo[d] = pb[at + d];
+        o.hi[d] = pb[at + 3 + d];
+        o.count *= uint32_t(o.hi[d] - o.lo[d]);
+      }
+      return o;
+    };
+    auto join = [&](const Box<T, D>& o) {
+      if (o.count == 0) return;
+      if (R.count == 0) {
+        R = o;
+        return;
+      }
+      R.count = 1;
+#pragma unroll
+      for (int d = 0; d < 3; ++d) {
+        R.lo[d] = min(R.lo[d], o.lo[d]);
+        R.hi[d] = max(R.hi[d], o.hi[d]);
         R.count *= uint32_t(R.hi[d] - R.lo[d]);
       }
+    };
+    bp = read(6);
+    join(bp);
+    if (hlbm) {
+      bs = read(12);
+      join(bs);
     }
     // (constant indices only: a box indexed per lane would be placed in LDS,
     // one copy per thread, halving the gather's occupancy)
     if (chunk == 0 && threadIdx.x == 0) {
 #pragma unroll
       for (int d = 0; d < 3; ++d) {
-        a.boxes[size_t(p) * 12 + d] = b.lo[d];
-        a.boxes[size_t(p) * 12 + 3 + d] = b.hi[d];
+        a.boxes[size_t(p) * kBoxInts + d] = b.lo[d];
+        a.boxes[size_t(p) * kBoxInts + 3 + d] = b.hi[d];
       }
     }
   }
-  if constexpr (LOCAL) lo.build(a, p, R, sweep);
   double acc[6] = {0, 0, 0, 0, 0, 0};
-  for (uint32_t k = chunk * blockDim.x + threadIdx.x; k < R.count;
-       k += a.blocks_per_particle * blockDim.x) {
-    int x[3];
-    box_cell<T, D>(R, k, x);
-    if (kCanSweep && sweep && !box_has<T, D>(b, x)) {
-      if (box_has<T, D>(bp, x) && !lo.held(a, p, x))
-        por[uint32_t(x[0]) + uint32_t(a.nx) * (uint32_t(x[1]) + uint32_t(a.ny) * uint32_t(x[2]))] = F(1);
-      continue;
-    }
+  // (uniform trip count: the block's list is built inside, behind the first
+  // cell's population loads, which do not need it)
+  bool listed = !LOCAL;
+  for (uint32_t k0 = chunk * blockDim.x; k0 < R.count; k0 += a.blocks_per_particle * blockDim.x) {
+    const uint32_t k = k0 + threadIdx.x;
+    const bool valid = k < R.count;
+    int x[3] = {R.lo[0], R.lo[1], R.lo[2]};
+    if (valid) box_cell<T, D>(R, k, x);
     T rel[3] = {T(0), T(0), T(0)};
     const T B = porosity_at<T, D>(P, x, eps, rel);
+    // every f_i at x and f_opp(i) at x + c_i first, all loads in flight at once
+    T fi[Q], fo[Q];
+    if constexpr (!fplbm) gather_pops<L, S, T>(a, x, fi, fo);
+    if (!listed) {
+      lo.build(a, p, R, sweep);
+      listed = true;
+    }
+    if (!valid) continue;
     const uint32_t c = uint32_t(x[0]) + uint32_t(a.nx) * (uint32_t(x[1]) + uint32_t(a.ny) * uint32_t(x[2]));
+    if (kCanSweep && sweep) {
+      if (hlbm && box_has<T, D>(bs, x)) {
+        for (int d = 0; d < D; ++d) static_cast<F*>(a.pn)[size_t(d) * a.N + c] = F(0);
+        static_cast<F*>(a.pd)[c] = F(0);
+      }
+      if (!box_has<T, D>(b, x)) {
+        if (box_has<T, D>(bp, x) && !lo.held(a, p, x)) por[c] = F(1);
+        continue;
+      }
+    }
     bool own_box, own_solid;
     if constexpr (LOCAL) {
       lo.test(a, p, x, !fplbm && B < T(1.0), eps, own_box, own_solid);
@@ -547,16 +681,6 @@ __global__ __launch_bounds__(256) void k_gather(ParticleArgs a) {
       continue;
     }
     if (B >= T(1.0)) continue;
-    // every f_i at x and f_opp(i) at x + c_i first, all loads in flight at once
-    T fi[Q], fo[Q];
-#pragma unroll
-    for (int i = 1; i < Q; ++i) {
-      fi[i] = pop_sel<L, S, T>(a, i, x[0], x[1], x[2], true);
-      int xn = x[0] + L::cx[i], yn = x[1] + L::cy[i], zn = x[2] + L::cz[i];
-      const bool ok = wrap(xn, a.nx, a.periodic & 1u) && wrap(yn, a.ny, a.periodic & 2u) &&
-                      wrap(zn, a.nz, a.periodic & 4u);
-      fo[i] = pop_sel<L, S, T>(a, L::opp[i], ok ? xn : x[0], ok ? yn : x[1], ok ? zn : x[2], ok);
-    }
     T mom[3] = {T(0.0), T(0.0), T(0.0)};
 #pragma unroll
     for (int i = 1; i < Q; ++i) {
@@ -916,7 +1040,7 @@ __global__ __launch_bounds__(64) void k_contact(ParticleArgs a) {
   }
   // the gather's box of this step becomes the previous box of the next
   if (a.boxes && a.fuse_finalize)
-    for (int k = 0; k < 6; ++k) a.boxes[size_t(s) * 12 + 6 + k] = a.boxes[size_t(s) * 12 + k];
+    for (int k = 0; k < 6; ++k) a.boxes[size_t(s) * kBoxInts + 6 + k] = a.boxes[size_t(s) * kBoxInts + k];
   // only this particle's record is written; other blocks read the snapshot
   // (fused) or only positions, rotations, masses and radii (not fused)
   for (int k = 0; k < D; ++k) me[PF_FORCE + k] = Fs[k];
@@ -976,14 +1100,14 @@ __global__ void k_integrate(ParticleArgs a) {
 __global__ void k_commit_boxes(int32_t* boxes, uint32_t n) {
   const uint32_t p = blockIdx.x * blockDim.x + threadIdx.x;
   if (p >= n) return;
-  for (int k = 0; k < 6; ++k) boxes[size_t(p) * 12 + 6 + k] = boxes[size_t(p) * 12 + k];
+  for (int k = 0; k < 6; ++k) boxes[size_t(p) * kBoxInts + 6 + k] = boxes[size_t(p) * kBoxInts + k];
 }
 
-// no previous boxes: every particle's lo = hi = 0
+// no previous and no stamped boxes: every particle's lo = hi = 0
 __global__ void k_clear_prev_boxes(int32_t* boxes, uint32_t n) {
   const uint32_t p = blockIdx.x * blockDim.x + threadIdx.x;
   if (p >= n) return;
-  for (int k = 0; k < 6; ++k) boxes[size_t(p) * 12 + 6 + k] = 0;
+  for (int k = 6; k < kBoxInts; ++k) boxes[size_t(p) * kBoxInts + k] = 0;
 }
 
 // ---------------------------------------------------------------- launchers
@@ -993,7 +1117,7 @@ static hipError_t couple_t(const ParticleArgs& a, hipStream_t s) {
   const bool scatter = a.porosity_mode == LBM_POROSITY_SCATTER;
   // one pass over the cells: PsmReset's porosity, the owners, HlbmReset's N
   // and D, FpLbmReset's force (the PSM sweep keeps the porosity without it)
-  const bool sweep = a.boxes != nullptr && scatter && !a.owner && !a.hlbm && !a.fplbm;
+  const bool sweep = a.boxes != nullptr && scatter && !a.owner && !a.fplbm;
   if (!sweep)
     hipLaunchKernelGGL((k_reset_cells<F>), dim3((N + 255) / 256), dim3(256), 0, s, (F*)a.por, a.owner,
                        a.hlbm ? (F*)a.pn : nullptr, a.hlbm ? (F*)a.pd : nullptr,
@@ -1042,13 +1166,14 @@ static hipError_t couple_l(int storage, const ParticleArgs& a, hipStream_t s) {
   return hipErrorInvalidValue;
 }
 
-hipError_t launch_sweep_reset(bool dbl, void* por, uint32_t N, int32_t* boxes, uint32_t n, hipStream_t s) {
+hipError_t launch_sweep_reset(bool dbl, int dims, void* por, void* pn, void* pd, uint32_t N, int32_t* boxes, uint32_t n,
+                              hipStream_t s) {
   if (dbl)
     hipLaunchKernelGGL((k_reset_cells<double>), dim3((N + 255) / 256), dim3(256), 0, s, (double*)por, nullptr,
-                       nullptr, nullptr, nullptr, N, 0, 1);
+                       (double*)pn, (double*)pd, nullptr, N, dims, 1);
   else
     hipLaunchKernelGGL((k_reset_cells<float>), dim3((N + 255) / 256), dim3(256), 0, s, (float*)por, nullptr,
-                       nullptr, nullptr, nullptr, N, 0, 1);
+                       (float*)pn, (float*)pd, nullptr, N, dims, 1);
   if (n > 0) hipLaunchKernelGGL(k_clear_prev_boxes, dim3((n + 255) / 256), dim3(256), 0, s, boxes, n);
   return hipGetLastError();
 }
