@@ -27,6 +27,7 @@ def _round_trip(lattice, storage, ext, seed):
 @pytest.mark.parametrize("lattice,storage,ext", [
     (abi.D2Q9, abi.F32, (3, 3)), (abi.D2Q9, abi.F64, (97, 31)),
     (abi.D2Q9, abi.F32, (87381, 1)), (abi.D2Q9, abi.F32, (87382, 1)),  # 4 bytes to either side of 1 MiB
+    (abi.D2Q9, abi.F32, (699050, 1)), (abi.D2Q9, abi.F32, (699051, 1)),  # and of 8 MiB
     (abi.D2Q9, abi.F32, (1023, 517)), (abi.D3Q19, abi.F64, (61, 67, 71)),
     (abi.D3Q19, abi.F16S, (257, 129, 131)), (abi.D3Q19, abi.F64, (129, 127, 131)),
 ])
