@@ -490,19 +490,72 @@ __global__ __launch_bounds__(256) void k_wgrad(WgradArgs a) {
 // pixels with one more on either side serve the three taps.  Both operands go
 // to LDS as they lie in memory (pixel by pixel, straight from the loads) and are
 // transposed on the way out (ds_read_b64_tr_b16: 16 lanes read 4 pixels x 16
-// channels and each gets the 4 pixels of its channel); the pixel pitches are odd
-// multiples of 32 bytes, so the 4 pixels of a read lie in different banks.
-// (That transposing write, 32 bits at a time, is most of k_wgrad's time.)
+// channels and each gets the 4 pixels of its channel), the tiles of a pixel
+// exchanged by wg_swap against bank conflicts.
 // Two buffers of kWgSteps K steps: the loads of one are in flight under the
-// MFMAs of the other.  Where a K step lies is scalar arithmetic; a load costs
+// MFMAs of the other.  At 256 x 256, batch 16, 96 -> 32 channels: 300 us by k_wgrad,
+// 167 us with the loads in flight waited for before the LDS reads (the compiler's
+// wait, see tr_read2) and conflicts in half of LDS' cycles, 161 us without the
+// conflicts, 134 us without the wait; 128 x 128, 160 -> 64: 174, 120, 114, 87 us.
+// Three buffers, or four steps to a buffer, are no faster: what bounds it now is
+// the pixels' way from L2 (each read for three dy and every 32 channels).  Where a K step lies is scalar arithmetic; a load costs
 // its thread an add and a select (with addresses worked out per thread and
 // load, their arithmetic bound the kernel).  Of the 6 x NC result tiles a
 // wavefront has 3 x NC/2.  The K steps and their pixels are k_wgrad's, so the
 // partial sums are its bits.
 constexpr int kWgSteps = 2;
+// Four transposing LDS reads of 8 bytes a lane (two operands of 8 pixels) at byte
+// addresses `at` plus OFF, or two (one operand), waited for before their results
+// are used.  In assembly because the compiler, which cannot tell the buffers apart,
+// waits before any LDS read for all loads to LDS that are in flight, and those of
+// the next K steps are meant to be.
+template <int OFF>
+__device__ __forceinline__ void tr_read2(const uint32_t (&p)[2], const uint32_t (&q)[2], bf16x8& a, bf16x8& b) {
+  u32x2 r0, r1, r2, r3;
+  asm volatile(
+      "ds_read_b64_tr_b16 %0, %4 offset:%8\n\t"
+      "ds_read_b64_tr_b16 %1, %5 offset:%8\n\t"
+      "ds_read_b64_tr_b16 %2, %6 offset:%8\n\t"
+      "ds_read_b64_tr_b16 %3, %7 offset:%8\n\t"
+      "s_waitcnt lgkmcnt(0)"
+      : "=&v"(r0), "=&v"(r1), "=&v"(r2), "=&v"(r3)
+      : "v"(p[0]), "v"(p[1]), "v"(q[0]), "v"(q[1]), "n"(OFF)
+      : "memory");
+  a = __builtin_bit_cast(bf16x8, u32x4{r0.x, r0.y, r1.x, r1.y});
+  b = __builtin_bit_cast(bf16x8, u32x4{r2.x, r2.y, r3.x, r3.y});
+}
+template <int OFF>
+__device__ __forceinline__ void tr_read1(const uint32_t (&p)[2], bf16x8& a) {
+  u32x2 r0, r1;
+  asm volatile(
+      "ds_read_b64_tr_b16 %0, %2 offset:%4\n\t"
+      "ds_read_b64_tr_b16 %1, %3 offset:%4\n\t"
+      "s_waitcnt lgkmcnt(0)"
+      : "=&v"(r0), "=&v"(r1)
+      : "v"(p[0]), "v"(p[1]), "n"(OFF)
+      : "memory");
+  a = __builtin_bit_cast(bf16x8, u32x4{r0.x, r0.y, r1.x, r1.y});
+}
+// Operands v[0 .. N) of one K step
+template <int OFF, int N>
+__device__ __forceinline__ void tr_read(const uint32_t (&at)[N][2], bf16x8 (&v)[N]) {
+#pragma unroll
+  for (int i = 0; i + 1 < N; i += 2) tr_read2<OFF>(at[i], at[i + 1], v[i], v[i + 1]);
+  if constexpr (N % 2 == 1) tr_read1<OFF>(at[N - 1], v[N - 1]);
+}
+// Which 32-byte tile of a pixel (of PT) stands where: tile t at t ^ wg_swap(pixel).
+// A transposing read takes 32 bytes of pixels r .. r + 3 and r + 8 .. r + 11 at a
+// time (half a wavefront), which then lie in all 64 banks.
+template <int PT>
+__device__ inline int wg_swap(int px) {
+  if (PT == 8) return (px & 3) | ((px >> 3 & 1) << 2);  // pixels 256 bytes apart
+  if (PT == 4) return (px >> 1 & 1) | ((px >> 3 & 1) << 1);
+  return px >> 3 & 1;
+}
 template <int NC>
 __global__ __launch_bounds__(256) void k_wgrad32(WgradArgs a, int splits) {
-  constexpr int PA = 6, PB = (NC | 1) * 2;    // pixel pitch in 16-byte chunks
+  constexpr int PT = (NC + 1) / 2 * 2;           // 16-channel tiles (32 bytes) of a pixel in LDS
+  constexpr int PA = 4, PB = 2 * PT;              // the same in 16-byte chunks
   constexpr int CA = 34 * PA, CS = CA + 32 * PB;  // chunks of a K step: of the input, of both
   constexpr int NT = (CS + 255) / 256, NH = (NC + 1) / 2;
   __shared__ u32x4 buf[2][kWgSteps][CS];
@@ -528,7 +581,8 @@ __global__ __launch_bounds__(256) void k_wgrad32(WgradArgs a, int splits) {
   for (int t = 0; t < NT; ++t) {
     const int i = tid + 256 * t;
     is_a[t] = i < CA;
-    const int px = is_a[t] ? i / PA : (i - CA) / PB, ch = is_a[t] ? i - px * PA : i - CA - px * PB;
+    const int px = is_a[t] ? i / PA : (i - CA) / PB, at_ = is_a[t] ? i - px * PA : i - CA - px * PB;
+    const int ch = at_ ^ (2 * (is_a[t] ? wg_swap<2>(px) : wg_swap<PT>(px)));  // (its tile, exchanged)
     const int c = (is_a[t] ? c0 : n0) + ch * 8;
     const bool ok = i < CS && ch < (is_a[t] ? 4 : 2 * NC) && c < (is_a[t] ? a.cin : N);
     gone[t] = !ok ? kNever : (!is_a[t] ? 0u : kRow | (px == 0 ? kLeft : 0u) | (px == 33 ? kRight : 0u));
@@ -562,15 +616,24 @@ __global__ __launch_bounds__(256) void k_wgrad32(WgradArgs a, int splits) {
       }
     }
   };
-  typedef short s16x4 __attribute__((ext_vector_type(4)));
-  using L4 = __attribute__((address_space(3))) s16x4;
-  // 8 pixels of a 16-channel operand: at, the lane's address of the first four
-  auto frag = [&](const uint16_t* at, int pitch) {
-    const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((L4*)at);
-    const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((L4*)(at + 4 * pitch * 8));
-    return __builtin_bit_cast(bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
-  };
   const int wm = wave & 1, wn = wave >> 1;
+  // where the lane finds the first and the second four of an operand's 8 pixels:
+  // byte addresses in the first buffer, of the input's tiles, then dpre's
+  uint32_t at[3 + NH][2];
+  const uint32_t lds0 = uint32_t(uintptr_t((__attribute__((address_space(3))) char*)&buf[0][0][0]));
+#pragma unroll
+  for (int e = 0; e < 2; ++e) {
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+      const int tile = wm * 3 + i, r = 8 * g + (j >> 2) + tile / 2 + 4 * e;  // tap dx = tile / 2, channels 16 (tile % 2) ..
+      at[i][e] = lds0 + r * PA * 16 + ((tile & 1) ^ wg_swap<2>(r)) * 32 + (j & 3) * 8;
+    }
+#pragma unroll
+    for (int n = 0; n < NH; ++n) {
+      const int r = 8 * g + (j >> 2) + 4 * e;
+      at[3 + n][e] = lds0 + CA * 16 + r * PB * 16 + ((wn * NH + n) ^ wg_swap<PT>(r)) * 32 + (j & 3) * 8;
+    }
+  }
   const bool bias = dy == 1 && c0 == 0 && wm == 1;  // row 9*cin: ones against dpre
   f32x4 acc[3][NH], accb[NH];
 #pragma unroll
@@ -587,27 +650,26 @@ __global__ __launch_bounds__(256) void k_wgrad32(WgradArgs a, int splits) {
     __builtin_amdgcn_s_waitcnt(0);
     __syncthreads();  // this buffer has arrived; no wave reads the other one any more
     if (k0 + kWgSteps < nk) load(b ^ 1);
+    uint32_t now[3 + NH][2];
 #pragma unroll
-    for (int ks = 0; ks < kWgSteps; ++ks) {
-      if (k0 + ks >= nk) break;
-      const uint16_t* lds = reinterpret_cast<const uint16_t*>(buf[b][ks]);
-      bf16x8 af[3], bf[NH];
+    for (int i = 0; i < 3 + NH; ++i)
 #pragma unroll
-      for (int i = 0; i < 3; ++i) {
-        const int tile = wm * 3 + i;  // tap dx = tile / 2, channels 16 (tile % 2) ..
-        af[i] = frag(lds + (8 * g + (j >> 2) + tile / 2) * PA * 8 + (tile & 1) * 16 + (j & 3) * 4, PA);
-      }
-#pragma unroll
-      for (int n = 0; n < NH; ++n)
-        if (wn * NH + n < NC)
-          bf[n] = frag(lds + CA * 8 + (8 * g + (j >> 2)) * PB * 8 + (wn * NH + n) * 16 + (j & 3) * 4, PB);
+      for (int e = 0; e < 2; ++e) now[i][e] = at[i][e] + (b ? kWgSteps * CS * 16 : 0);
+    auto k_step = [&](const bf16x8 (&v)[3 + NH]) {
 #pragma unroll
       for (int n = 0; n < NH; ++n) {
         if (wn * NH + n >= NC) continue;
 #pragma unroll
-        for (int i = 0; i < 3; ++i) acc[i][n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bf[n], af[i], acc[i][n], 0, 0, 0);
-        if (bias) accb[n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bf[n], ones, accb[n], 0, 0, 0);
+        for (int i = 0; i < 3; ++i) acc[i][n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(v[3 + n], v[i], acc[i][n], 0, 0, 0);
+        if (bias) accb[n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(v[3 + n], ones, accb[n], 0, 0, 0);
       }
+    };
+    bf16x8 v[3 + NH];
+    tr_read<0>(now, v);
+    k_step(v);
+    if (k0 + 1 < nk) {
+      tr_read<CS * 16>(now, v);
+      k_step(v);
     }
   }
   float* out = a.partial + size_t(s) * Mx * N;
@@ -631,8 +693,8 @@ hipError_t launch_wgrad_n(const WgradArgs& a, int splits, hipStream_t s) {
   const size_t px = size_t(a.B) * a.H * a.W;
   // Fewer channels than its 32 leave k_wgrad32's tiles mostly empty: 49 us for 41
   // at 256 x 256 from 8 channels.  From 32 on it is the faster one there (96 -> 32
-  // channels 300 -> 167 us, 32 -> 32 128 -> 71 us, 32 -> 3 110 -> 57 us) and about
-  // even where rows are one K step long (160 channels at 32 x 32: 27 us both).
+  // channels 300 -> 134 us, 32 -> 32 128 -> 63 us, 32 -> 3 110 -> 45 us) and down to
+  // rows of one K step (160 channels at 32 x 32: 27 -> 19 us).
   if (a.cin > 16 && a.W % 32 == 0 && act_small(a.in, px) && act_small(a.dpre, px))
     hipLaunchKernelGGL(k_wgrad32<NC>, dim3((splits + 7) / 8 * 8 * 3 * ((a.cin + 31) / 32) * cols), dim3(256), 0, s, a,
                        splits);
@@ -655,30 +717,44 @@ hipError_t launch_wgrad(const WgradArgs& a, int splits, hipStream_t s) {
 // unpadded Cout); row 9*cin is the bias, which follows the weights in the
 // flat parameter layout.  A block takes 64 consecutive outputs: four groups
 // of 64 threads add the splits k = g, g+4, ..., then the four sums are added
-// in group order (a fixed order: training repeats bit for bit).
-__global__ __launch_bounds__(256) void k_wreduce(const float* partial, int splits, int Mw, int cpad, int cr,
-                                                 float* grad) {
+// in group order (a fixed order: training repeats bit for bit).  One launch for
+// all layers, each with partial tiles of its own: a layer alone has 14 to 900
+// blocks whose threads add up to 256 values one after the other, 113 us a step
+// in twelve launches, 72 us in one.
+struct WredLayer {
+  const float* partial;
+  float* grad;
+  int splits, Mw, cpad, cr;
+  unsigned end;  // of this layer's blocks
+};
+struct WredArgs {
+  WredLayer layer[12];
+};
+__global__ __launch_bounds__(256) void k_wreduce(WredArgs a) {
   __shared__ float part[4][64];
+  int q = 0;
+  while (blockIdx.x >= a.layer[q].end) ++q;
+  const WredLayer& L = a.layer[q];
   const int gq = threadIdx.x >> 6, l = threadIdx.x & 63;
-  const int i = blockIdx.x * 64 + l;
-  const bool ok = i < (Mw + 1) * cr;
-  const int m = ok ? i / cr : 0, n = ok ? i - m * cr : 0;
+  const int i = int(blockIdx.x - (q > 0 ? a.layer[q - 1].end : 0u)) * 64 + l;
+  const bool ok = i < (L.Mw + 1) * L.cr;
+  const int m = ok ? i / L.cr : 0, n = ok ? i - m * L.cr : 0;
   // four running sums per thread (splits gq + 4(4i + u), u = 0..3) keep
   // four loads in flight; combined in a fixed order
   float su[4] = {0.f, 0.f, 0.f, 0.f};
   if (ok) {
-    const size_t stride = size_t(Mw + 8) * cpad;
-    const float* src = partial + size_t(m) * cpad + n;
+    const size_t stride = size_t(L.Mw + 8) * L.cpad;
+    const float* src = L.partial + size_t(m) * L.cpad + n;
     int k = gq;
-    for (; k + 12 < splits; k += 16) {
+    for (; k + 12 < L.splits; k += 16) {
 #pragma unroll
       for (int u = 0; u < 4; ++u) su[u] += src[size_t(k + 4 * u) * stride];
     }
-    for (int u = 0; k < splits; k += 4, ++u) su[u] += src[size_t(k) * stride];
+    for (int u = 0; k < L.splits; k += 4, ++u) su[u] += src[size_t(k) * stride];
   }
   part[gq][l] = (su[0] + su[1]) + (su[2] + su[3]);
   __syncthreads();
-  if (gq == 0 && ok) grad[i] = ((part[0][l] + part[1][l]) + part[2][l]) + part[3][l];
+  if (gq == 0 && ok) L.grad[i] = ((part[0][l] + part[1][l]) + part[2][l]) + part[3][l];
 }
 
 // 8 channels (16 bytes, 16-byte aligned: channel offsets and row pitches are
@@ -847,7 +923,7 @@ struct WconvLayer {
   const float* wm;
   uint16_t *wb, *wt;
   int cin, cr, cpad;
-  size_t end;  // of this layer's elements in the launch
+  size_t end;  // in 16-byte units: of this layer's elements in the launch
 };
 struct WconvArgs {
   WconvLayer layer[12];
@@ -856,25 +932,31 @@ __host__ __device__ inline size_t conv_elements(int cin, int N) {
   return size_t(conv_steps(cin)) * conv_tiles(N) * 512;
 }
 __global__ void k_wconvert(WconvArgs a) {
+  // a thread writes a lane's 16 bytes: one tap's 8 channels in a row, while 16
+  // lanes read neighbouring floats (one element a thread: 18 us a step, not 9)
   const size_t step = size_t(gridDim.x) * 256;
   for (size_t i = size_t(blockIdx.x) * 256 + threadIdx.x; i < a.layer[11].end; i += step) {
     int k = 0;
     while (i >= a.layer[k].end) ++k;
     const WconvLayer& L = a.layer[k];
     size_t e = i - (k > 0 ? a.layer[k - 1].end : 0);
-    const size_t nf = conv_elements(L.cin, L.cpad);
+    const size_t nf = conv_elements(L.cin, L.cpad) / 8;
     const bool fwd = e < nf;
     if (!fwd) e -= nf;
     const int ci = fwd ? L.cin : L.cpad, N = fwd ? L.cpad : L.cin, nt = conv_tiles(N);
-    const int lane = int(e >> 3) & 63, frag = int(e >> 9), t = frag % nt;
-    const int kk = frag / nt * 32 + (lane >> 4) * 8 + int(e & 7), tap = kk / ci, c = kk - tap * ci;
+    const int lane = int(e & 63), frag = int(e >> 6), t = frag % nt;
+    const int kk = frag / nt * 32 + (lane >> 4) * 8, tap = kk / ci, c = kk - tap * ci;
     const int n = conv_channel(conv_nc(N), t, lane & 15);
-    uint16_t v = 0;
+    uint32_t v[4] = {0u, 0u, 0u, 0u};
     if (tap < 9 && n < N) {
-      const int in = fwd ? c : n, out = fwd ? n : c;
-      if (out < L.cr) v = f2bf(L.wm[(size_t(fwd ? tap : 8 - tap) * L.cin + in) * L.cr + out]);
+      const float* wm = L.wm + size_t(fwd ? tap : 8 - tap) * L.cin * L.cr;
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        const int in = fwd ? c + j : n, out = fwd ? n : c + j;
+        if (out < L.cr) v[j / 2] |= uint32_t(f2bf(wm[size_t(in) * L.cr + out])) << (j & 1 ? 16 : 0);
+      }
     }
-    (fwd ? L.wb : L.wt)[e] = v;
+    reinterpret_cast<uint4*>(fwd ? L.wb : L.wt)[e] = make_uint4(v[0], v[1], v[2], v[3]);
   }
 }
 
@@ -893,11 +975,10 @@ __global__ void k_standardize(float* t, size_t n, float m0, float m1, float m2, 
 // bytes a pixel.  (Laid out by the host this was 16 of the 20 ms of 16
 // predictions of 256 x 256.)
 __global__ void k_features(const uint8_t* flags, const uint32_t* tab, int B, int H, int W, uint16_t* x) {
-  const size_t i = size_t(blockIdx.x) * blockDim.x + threadIdx.x, HW = size_t(H) * W;
+  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x, HW = uint32_t(H) * uint32_t(W);
   if (i >= B * HW) return;
-  const size_t b = i / HW;
-  const int r = int(i - b * HW), py = r / W, px = r - py * W;
-  const uint32_t* per = tab + H + W + b * (W + 1);
+  const uint32_t b = i / HW, r = i - b * HW, py = r / uint32_t(W), px = r - py * uint32_t(W);
+  const uint32_t* per = tab + H + W + size_t(b) * (W + 1);
   const uint32_t row = tab[py], col = tab[H + px], own = per[0], at = per[1 + px];
   const uint32_t open = flags[i] >= 2 ? 0x3f80u : 0u;
   // channels 0 .. 7: open, speed | tau, profile | x, y | pressure, blockage
@@ -907,14 +988,14 @@ __global__ void k_features(const uint8_t* flags, const uint32_t* tab, int B, int
 
 __global__ void k_gather(const uint16_t* xs, const float* ts, const uint8_t* ms, const uint32_t* idx, int B, int HW,
                          uint16_t* x, float* t, uint8_t* m) {
-  const size_t i = size_t(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (i >= size_t(B) * HW) return;
-  const int b = int(i / HW), p = int(i % HW);
+  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;  // (the batch's pixels fit an int)
+  if (i >= uint32_t(B) * uint32_t(HW)) return;
+  const uint32_t b = i / uint32_t(HW), p = i - b * uint32_t(HW);
   const size_t src = size_t(idx[b]) * HW + p;
-  *reinterpret_cast<uint4*>(x + i * 8) = *reinterpret_cast<const uint4*>(xs + src * 8);
-  t[i * 3 + 0] = ts[src * 3 + 0];
-  t[i * 3 + 1] = ts[src * 3 + 1];
-  t[i * 3 + 2] = ts[src * 3 + 2];
+  *reinterpret_cast<uint4*>(x + size_t(i) * 8) = *reinterpret_cast<const uint4*>(xs + src * 8);
+  t[size_t(i) * 3 + 0] = ts[src * 3 + 0];
+  t[size_t(i) * 3 + 1] = ts[src * 3 + 1];
+  t[size_t(i) * 3 + 2] = ts[src * 3 + 2];
   m[i] = ms[src];
 }
 
@@ -952,6 +1033,7 @@ double rho_unit(double u_max) { return 3.0 * u_max * u_max; }
 struct Layer {
   int cin, cr, cpad;  // input channels, output channels (real / padded to 8)
   size_t w_off, b_off;
+  size_t p_off = 0;  // of its partial weight-gradient tiles
   uint16_t *wb = nullptr, *wt = nullptr;
   int relu;
   int level;
@@ -977,7 +1059,6 @@ struct lbm_net {
   uint8_t* msk = nullptr;
   uint32_t* ftab = nullptr;  // upload_features' words
   float* partial = nullptr;
-  size_t partial_n = 0;
   double* lpartial = nullptr;
   double* dloss = nullptr;
   float* dlosses = nullptr;
@@ -1060,11 +1141,14 @@ Act act(uint16_t* p, int ld, int off = 0) { return Act{p, ld, off}; }
 #define LBMNET_WGRAD_BLOCKS 1024
 #endif
 constexpr int kWgradBlocks = LBMNET_WGRAD_BLOCKS;
-void wgrad_shape(const lbm_net* n, const Layer& L, int B, int& splits, int& chunk) {
-  const int M = B * H_(n, L.level) * W_(n, L.level);
+int wgrad_most_splits(const Layer& L, int M) {  // no fewer pixels have more
   const int bn = 16 * wgrad_nc(L.cpad);
   const int tiles = ((9 * L.cin + 8 + BM - 1) / BM) * ((L.cpad + bn - 1) / bn);
-  splits = std::max(1, std::min(kWgradBlocks / std::max(1, tiles), (M + 255) / 256));
+  return std::max(1, std::min(kWgradBlocks / std::max(1, tiles), (M + 255) / 256));
+}
+void wgrad_shape(const lbm_net* n, const Layer& L, int B, int& splits, int& chunk) {
+  const int M = B * H_(n, L.level) * W_(n, L.level);
+  splits = wgrad_most_splits(L, M);
   chunk = ((M + splits - 1) / splits + BK - 1) / BK * BK;
   splits = (M + chunk - 1) / chunk;
 }
@@ -1090,20 +1174,16 @@ lbm_status conv(lbm_net* n, int li, int B, Act in, Act out, float* outf) {
   return LBM_OK;
 }
 
-// Backward of layer li given its pre-activation gradient dpre: weight and
-// bias gradients into n->g, and (if dx.p) the input gradient, masked by
+// Backward of layer li given its pre-activation gradient dpre: the partial
+// tiles of its weight and bias gradients (reduce_gradients), and (if dx.p) the input gradient, masked by
 // (in > 0) when mask_in.
 lbm_status conv_bwd(lbm_net* n, int li, int B, Act in, Act dpre, Act dx, bool mask_in) {
   const Layer& L = n->layers[li];
   const int H = H_(n, L.level), W = W_(n, L.level);
   int splits, chunk;
   wgrad_shape(n, L, B, splits, chunk);
-  WgradArgs wa{B, H, W, L.cin, L.cpad, in, dpre, n->partial, chunk};
+  WgradArgs wa{B, H, W, L.cin, L.cpad, in, dpre, n->partial + L.p_off, chunk};
   NET_TRY(launch_wgrad(wa, splits, n->stream));
-  const int Mw = 9 * L.cin;
-  hipLaunchKernelGGL(k_wreduce, dim3(((Mw + 1) * L.cr + 63) / 64), dim3(256), 0, n->stream, n->partial, splits, Mw,
-                     L.cpad, L.cr, n->g + L.w_off);
-  NET_TRY(hipGetLastError());
   if (dx.p) {
     ConvArgs a{};
     a.B = B;
@@ -1199,6 +1279,22 @@ lbm_status loss_fwd(lbm_net* n, int B, double nf, double* dloss, float* dlossf) 
   return LBM_OK;
 }
 
+// Every layer's weight and bias gradient into n->g.
+lbm_status reduce_gradients(lbm_net* n, int B) {
+  WredArgs a{};
+  unsigned end = 0;
+  for (int k = 0; k < 12; ++k) {
+    const Layer& L = n->layers[k];
+    int splits, chunk;
+    wgrad_shape(n, L, B, splits, chunk);
+    end += unsigned(((9 * L.cin + 1) * L.cr + 63) / 64);
+    a.layer[k] = WredLayer{n->partial + L.p_off, n->g + L.w_off, splits, 9 * L.cin, L.cpad, L.cr, end};
+  }
+  hipLaunchKernelGGL(k_wreduce, dim3(end), dim3(256), 0, n->stream, a);
+  NET_TRY(hipGetLastError());
+  return LBM_OK;
+}
+
 lbm_status backward(lbm_net* n, int B) {
   const int* w = n->cfg.widths;
   const int cw[3] = {w[1] + w[0], w[2] + w[1], w[3] + w[2]};
@@ -1221,7 +1317,7 @@ lbm_status backward(lbm_net* n, int B) {
   NS(pool_bwd(n, 0, B, act(n->gpool[1], w[0]), act(n->gcat[0], cw[0], w[1]), act(n->cat[0], cw[0], w[1]), w[0]));
   NS(conv_bwd(n, 1, B, act(n->a[0], w[0]), act(n->gcat[0], cw[0], w[1]), act(n->ga[0], w[0]), true));
   NS(conv_bwd(n, 0, B, act(n->x, 8), act(n->ga[0], w[0]), none, false));
-  return LBM_OK;
+  return reduce_gradients(n, B);
 }
 
 lbm_status refresh_weights(lbm_net* n) {
@@ -1229,7 +1325,7 @@ lbm_status refresh_weights(lbm_net* n) {
   size_t end = 0;
   for (int k = 0; k < 12; ++k) {
     const Layer& L = n->layers[k];
-    end += conv_elements(L.cin, L.cpad) + conv_elements(L.cpad, L.cin);
+    end += (conv_elements(L.cin, L.cpad) + conv_elements(L.cpad, L.cin)) / 8;
     a.layer[k] = WconvLayer{n->w + L.w_off, L.wb, L.wt, L.cin, L.cr, L.cpad, end};
   }
   hipLaunchKernelGGL(k_wconvert, dim3(unsigned(std::min<size_t>(blocks_for(end), 1 << 20))), dim3(256), 0, n->stream, a);
@@ -1389,14 +1485,12 @@ lbm_status create_impl(lbm_net* n) {
   NS(dalloc(&n->t, level_pixels(n, 0) * 3));
   NS(dalloc(&n->msk, level_pixels(n, 0)));
   NS(dalloc(&n->ftab, feature_words(n->cfg, c.batch)));
-  size_t pmax = 0;
-  for (const Layer& L : n->layers) {
-    int splits, chunk;
-    wgrad_shape(n, L, c.batch, splits, chunk);
-    pmax = std::max(pmax, size_t(splits) * (9 * L.cin + 8) * L.cpad);
+  size_t partial = 0;
+  for (Layer& L : n->layers) {
+    L.p_off = partial;
+    partial += size_t(wgrad_most_splits(L, int(level_pixels(n, L.level)))) * (9 * L.cin + 8) * L.cpad;
   }
-  n->partial_n = pmax;
-  NS(dalloc(&n->partial, pmax));
+  NS(dalloc(&n->partial, partial));
   NS(dalloc(&n->lpartial, size_t(blocks_for(level_pixels(n, 0)))));
   NS(dalloc(&n->dloss, 1));
   const size_t HW = size_t(c.height) * c.width;
