@@ -87,13 +87,22 @@ __device__ inline uint4 load_tap(const Act& s, int H, int W, int b, int y, int x
 }
 
 // 16-channel tiles per conv block for N output channels: the widest block of
-// at most 128 channels that divides N (N = 8, the output layer, takes 32)
+// at most 160 channels that divides N (N = 8, the output layer, takes 32).  160 in
+// one block read the pixels once, not twice: 64 -> 160 channels at 128 x 128 106 ->
+// 82 us.
 __host__ __device__ inline int conv_nc(int N) {
-  const int nc[5] = {8, 6, 5, 4, 2};
-  for (int k = 0; k < 5; ++k)
+  const int nc[6] = {10, 8, 6, 5, 4, 2};
+  for (int k = 0; k < 6; ++k)
     if (N % (16 * nc[k]) == 0) return nc[k];
   return 2;
 }
+// Wavefronts of a conv block that share its pixels and split its tiles.  Two halve
+// what the block reads of its weights, which comes through L1 at half LDS' rate
+// (with one, twice the time of the MFMAs): at 256 x 256, 32 -> 96 channels 168 -> 138
+// us, at 128 x 128 160 -> 64 77 -> 65 us, at 64 x 64 256 -> 96 65 -> 53 us.  Of two tiles
+// each wavefront keeps both: its 16-byte stores are worth more (8 -> 32 channels 30
+// us for 32).
+__host__ __device__ constexpr int conv_wn(int nc) { return nc >= 4 && nc % 2 == 0 ? 2 : 1; }
 // Weight fragments of a conv GEMM: per K step of 32 and 16-channel tile, the
 // 64 lanes' 16-byte MFMA operands in lane order, so a wavefront loads one as
 // 1 KiB in a row.  Lane l holds k = 8 (l / 16) .. + 7 of row l % 16.
@@ -120,16 +129,16 @@ constexpr int kPatchW = 18;  // 16 pixels and the halo
 // of the activation instead of one per tap, one barrier instead of one per K
 // step), and the nine taps read them there, each 16-pixel operand at its own
 // shift.  Pixels lie 2*cin + 16 bytes apart.  The weights come as ready
-// fragments from L1/L2, so they need no LDS either.  A wavefront has MT rows of
-// pixels and all NC tiles: per K step MT operands from LDS and NC from L1 for
-// MT*NC MFMAs.  The weights are the first operand: a lane's results are then 8
+// fragments from L1/L2, so they need no LDS either.  A wavefront has RT rows of
+// pixels and NW tiles (conv_wn): per K step RT operands from LDS and NW from L1 for
+// RT*NW MFMAs.  The weights are the first operand: a lane's results are then 8
 // consecutive channels of one pixel, stored as they are.  Batch of 16 images of
 // 256 x 256, per layer, against 128-pixel tiles gathered tap by tap through two
 // LDS buffers: 96 -> 32 channels 237 -> 110 us, 32 -> 32 79 -> 42 us, at 32 x 32
-// 96 -> 160 and 160 -> 160 channels 33 and 46 -> 16 and 22 us.  What bounds it
+// 96 -> 160 and 160 -> 160 channels 33 and 46 -> 16 and 21 us.  What bounds it
 // then: the many-channel layers the MFMA issue (96 -> 32: 58 GFLOP, 42 us at the
 // card's matrix-product rate) and LDS reads, the few-channel ones memory; the
-// input gradient of 96 channels at 256 x 256 (184 us, as before) the 400 MB of
+// input gradient of 96 channels at 256 x 256 (178 -> 138 us) the 400 MB of
 // its mask and result.
 // MODE 0: cin a multiple of 32 (a K step lies in one tap); 1: any cin (each
 // quarter of the lanes finds its own tap); 2: as 1, with the pixels read from
@@ -137,12 +146,15 @@ constexpr int kPatchW = 18;  // 16 pixels and the halo
 template <int NC, int MT, int MODE>
 __global__ __launch_bounds__(256) void k_conv(ConvArgs a) {
   extern __shared__ u32x4 patch[];
+  // wavefronts along the pixel rows and along the tiles, and what each has of both
+  constexpr int WN = conv_wn(NC), NW = NC / WN, RT = MT * WN;
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, g = lane >> 4, px = lane & 15;
   const int tx = (a.W + 15) / 16, ty = (a.H + 4 * MT - 1) / (4 * MT);
   const int bx = blockIdx.x % tx, by = blockIdx.x / tx % ty, b = blockIdx.x / (tx * ty);
   const int x0 = bx * 16, y0 = by * 4 * MT;
   const int c8 = a.cin / 8, sp = c8 + 1;  // pixel pitch in 16-byte units
-  const int nk = conv_steps(a.cin), nt = conv_tiles(a.cout), t0 = blockIdx.y * NC;
+  const int wm = wave / WN, wn = wave % WN;
+  const int nk = conv_steps(a.cin), nt = conv_tiles(a.cout), t0 = blockIdx.y * NC + wn * NW;
   const int zat = c8;  // MODE 1: a chunk of zeros (the first pixel's padding)
   if (MODE != 2) {
     // straight to LDS, 1 KiB a wavefront and instruction, so that the whole
@@ -169,21 +181,21 @@ __global__ __launch_bounds__(256) void k_conv(ConvArgs a) {
     __syncthreads();
   }
   // what the results will need of the layer's input, in flight under the MFMAs
-  constexpr int NP = (NC + 1) / 2;
+  constexpr int NP = (NW + 1) / 2;
   const int x = x0 + px;
-  auto pixel = [&](int r) { return (size_t(b) * a.H + (y0 + wave * MT + r)) * a.W + x; };
-  auto inside = [&](int r) { return y0 + wave * MT + r < a.H && x < a.W; };
+  auto pixel = [&](int r) { return (size_t(b) * a.H + (y0 + wm * RT + r)) * a.W + x; };
+  auto inside = [&](int r) { return y0 + wm * RT + r < a.H && x < a.W; };
   // a pair's first channel in this lane
-  auto channel = [&](int p) { return 16 * (t0 + 2 * p) + (2 * p + 1 < NC ? 8 : 4) * g; };
-  u32x4 mk[MT][NP];
+  auto channel = [&](int p) { return 16 * (t0 + 2 * p) + (2 * p + 1 < NW ? 8 : 4) * g; };
+  u32x4 mk[RT][NP];
   if (a.mask.p) {
     const auto mp = (const __attribute__((address_space(1))) uint16_t*)a.mask.p + a.mask.off;
 #pragma unroll
-    for (int r = 0; r < MT; ++r)
+    for (int r = 0; r < RT; ++r)
 #pragma unroll
       for (int p = 0; p < NP; ++p) {
         const auto at = mp + (inside(r) ? pixel(r) * a.mask.ld : size_t(0)) + (channel(p) < a.cout ? channel(p) : 0);
-        if (2 * p + 1 < NC) {
+        if (2 * p + 1 < NW) {
           mk[r][p] = *(const __attribute__((address_space(1))) u32x4*)at;
         } else {
           const auto t = *(const __attribute__((address_space(1))) u32x2*)at;
@@ -191,19 +203,19 @@ __global__ __launch_bounds__(256) void k_conv(ConvArgs a) {
         }
       }
   }
-  f32x4 acc[MT][NC];
+  f32x4 acc[RT][NW];
 #pragma unroll
-  for (int r = 0; r < MT; ++r)
+  for (int r = 0; r < RT; ++r)
 #pragma unroll
-    for (int c = 0; c < NC; ++c) acc[r][c] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int c = 0; c < NW; ++c) acc[r][c] = f32x4{0.f, 0.f, 0.f, 0.f};
   const auto wp = (const __attribute__((address_space(1))) u32x4*)a.w + size_t(t0) * 64 + lane;
-  const int base = (wave * MT * kPatchW + px) * sp + (MODE == 0 ? g : 0);
+  const int base = (wm * RT * kPatchW + px) * sp + (MODE == 0 ? g : 0);
   int tap = 0, c = 0;  // MODE 0: the K step's tap and first 8-channel chunk
-  auto mma = [&](const u32x4 (&w)[NC], const u32x4 (&p)[MT]) {
+  auto mma = [&](const u32x4 (&w)[NW], const u32x4 (&p)[RT]) {
 #pragma unroll
-    for (int r = 0; r < MT; ++r)
+    for (int r = 0; r < RT; ++r)
 #pragma unroll
-      for (int n = 0; n < NC; ++n)
+      for (int n = 0; n < NW; ++n)
         acc[r][n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, w[n]),
                                                             __builtin_bit_cast(bf16x8, p[r]), acc[r][n], 0, 0, 0);
   };
@@ -211,18 +223,18 @@ __global__ __launch_bounds__(256) void k_conv(ConvArgs a) {
     // nk = 9 * cin / 32 is a multiple of 3: three K steps per turn, the
     // weights of each loaded a whole turn ahead (the last turn's loads read
     // the fragments' padding)
-    u32x4 wf[3][NC];
+    u32x4 wf[3][NW];
 #pragma unroll
     for (int d = 0; d < 3; ++d)
 #pragma unroll
-      for (int n = 0; n < NC; ++n) wf[d][n] = wp[(d * nt + n) * 64];
+      for (int n = 0; n < NW; ++n) wf[d][n] = wp[(d * nt + n) * 64];
     for (int k = 0; k < nk; k += 3) {
 #pragma unroll
       for (int d = 0; d < 3; ++d) {
-        u32x4 pf[MT];
+        u32x4 pf[RT];
         const int off = base + (tap / 3 * kPatchW + tap % 3) * sp + c;
 #pragma unroll
-        for (int r = 0; r < MT; ++r) pf[r] = patch[off + r * kPatchW * sp];
+        for (int r = 0; r < RT; ++r) pf[r] = patch[off + r * kPatchW * sp];
         c += 4;
         if (c == c8) {
           c = 0;
@@ -230,22 +242,22 @@ __global__ __launch_bounds__(256) void k_conv(ConvArgs a) {
         }
         mma(wf[d], pf);
 #pragma unroll
-        for (int n = 0; n < NC; ++n) wf[d][n] = wp[size_t((k + 3 + d) * nt + n) * 64];
+        for (int n = 0; n < NW; ++n) wf[d][n] = wp[size_t((k + 3 + d) * nt + n) * 64];
       }
     }
   } else {
     for (int k = 0; k < nk; ++k) {
-      u32x4 wf[NC], pf[MT];
+      u32x4 wf[NW], pf[RT];
 #pragma unroll
-      for (int n = 0; n < NC; ++n) wf[n] = wp[size_t(k * nt + n) * 64];
+      for (int n = 0; n < NW; ++n) wf[n] = wp[size_t(k * nt + n) * 64];
       const int o = 4 * k + g, tp = o / c8, ch = o - tp * c8;  // this lane's tap and 8-channel chunk
       const bool in = tp < 9;
 #pragma unroll
-      for (int r = 0; r < MT; ++r) {
+      for (int r = 0; r < RT; ++r) {
         if (MODE == 1) {
           pf[r] = patch[in ? base + (r * kPatchW + tp / 3 * kPatchW + tp % 3) * sp + ch : zat];
         } else {
-          const int y = y0 + wave * MT + r, x = x0 + px;
+          const int y = y0 + wm * RT + r, x = x0 + px;
           const uint4 v = (in && y < a.H && x < a.W) ? load_tap(a.in, a.H, a.W, b, y, x, tp, ch * 8)
                                                      : make_uint4(0u, 0u, 0u, 0u);
           pf[r] = u32x4{v.x, v.y, v.z, v.w};
@@ -257,14 +269,14 @@ __global__ __launch_bounds__(256) void k_conv(ConvArgs a) {
   // 8 channels of a pixel per lane and store
 #pragma unroll
   for (int p = 0; p < NP; ++p) {
-    const bool pair = 2 * p + 1 < NC;
+    const bool pair = 2 * p + 1 < NW;
     const int ch = channel(p);
     if (ch >= a.cout) continue;
     float bias[8];
 #pragma unroll
     for (int j = 0; j < 8; ++j) bias[j] = (a.bias && ch + j < a.bias_n && (pair || j < 4)) ? a.bias[ch + j] : 0.f;
 #pragma unroll
-    for (int r = 0; r < MT; ++r) {
+    for (int r = 0; r < RT; ++r) {
       if (!inside(r)) continue;
       const size_t m = pixel(r);
       float v[8];
@@ -327,6 +339,7 @@ hipError_t launch_conv_n(const ConvArgs& a, hipStream_t s) {
 
 hipError_t launch_conv(const ConvArgs& a, hipStream_t s) {
   switch (conv_nc(a.cout)) {
+    case 10: return launch_conv_n<10>(a, s);
     case 8: return launch_conv_n<8>(a, s);
     case 6: return launch_conv_n<6>(a, s);
     case 5: return launch_conv_n<5>(a, s);
@@ -946,7 +959,7 @@ __global__ void k_wconvert(WconvArgs a) {
     const int ci = fwd ? L.cin : L.cpad, N = fwd ? L.cpad : L.cin, nt = conv_tiles(N);
     const int lane = int(e & 63), frag = int(e >> 6), t = frag % nt;
     const int kk = frag / nt * 32 + (lane >> 4) * 8, tap = kk / ci, c = kk - tap * ci;
-    const int n = conv_channel(conv_nc(N), t, lane & 15);
+    const int n = conv_channel(conv_nc(N) / conv_wn(conv_nc(N)), t, lane & 15);
     uint32_t v[4] = {0u, 0u, 0u, 0u};
     if (tap < 9 && n < N) {
       const float* wm = L.wm + size_t(fwd ? tap : 8 - tap) * L.cin * L.cr;
