@@ -199,7 +199,8 @@ enum PartField {
 };
 
 hipError_t launch_psm_couple(int lattice, int storage, const ParticleArgs& a, hipStream_t s);
-// Porosity 1 in every cell and every particle's previous box empty: the
+// Porosity 1 in every cell (with HLBM's fields: N = D = 0 too) and every particle's
+// previous and stamped box empty: the
 // state from which the gathers keep the porosity without a per-cell reset
 hipError_t launch_sweep_reset(bool dbl, int dims, void* por, void* pn, void* pd, uint32_t N, int32_t* boxes, uint32_t n,
                               hipStream_t s);

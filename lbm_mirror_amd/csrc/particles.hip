@@ -1,8 +1,9 @@
 // Particle coupling kernels.
 //
 // One PSM coupling pass (lbm_psm_couple) is, in launch order:
-//   k_reset_cells porosity := 1 (PsmReset, psm.hpp:20-32), owners := 0, HLBM N, D := 0,
-//                FPLBM force := 0
+//   k_reset_cells [FPLBM, product mode, more than kLocalOwnerMax particles; else the
+//                gather sweeps] porosity := 1 (PsmReset, psm.hpp:20-32), owners := 0,
+//                HLBM N, D := 0, FPLBM force := 0
 //   k_owner      [more than kLocalOwnerMax particles] per particle and AABB
 //                cell: which particle a serial loop over particles would have
 //                written last (highest index), for the porosity and for the
@@ -614,24 +615,10 @@ __global__ __launch_bounds__(256) void k_gather(ParticleArgs a) {
     }
   }
   double acc[6] = {0, 0, 0, 0, 0, 0};
-  // (uniform trip count: the block's list is built inside, behind the first
-  // cell's population loads, which do not need it)
-  bool listed = !LOCAL;
-  for (uint32_t k0 = chunk * blockDim.x; k0 < R.count; k0 += a.blocks_per_particle * blockDim.x) {
-    const uint32_t k = k0 + threadIdx.x;
-    const bool valid = k < R.count;
-    int x[3] = {R.lo[0], R.lo[1], R.lo[2]};
-    if (valid) box_cell<T, D>(R, k, x);
-    T rel[3] = {T(0), T(0), T(0)};
-    const T B = porosity_at<T, D>(P, x, eps, rel);
-    // every f_i at x and f_opp(i) at x + c_i first, all loads in flight at once
-    T fi[Q], fo[Q];
-    if constexpr (!fplbm) gather_pops<L, S, T>(a, x, fi, fo);
-    if (!listed) {
-      lo.build(a, p, R, sweep);
-      listed = true;
-    }
-    if (!valid) continue;
+  if constexpr (LOCAL) lo.build(a, p, R, sweep);
+  for (uint32_t k = chunk * blockDim.x + threadIdx.x; k < R.count; k += a.blocks_per_particle * blockDim.x) {
+    int x[3];
+    box_cell<T, D>(R, k, x);
     const uint32_t c = uint32_t(x[0]) + uint32_t(a.nx) * (uint32_t(x[1]) + uint32_t(a.ny) * uint32_t(x[2]));
     if (kCanSweep && sweep) {
       if (hlbm && box_has<T, D>(bs, x)) {
@@ -643,6 +630,8 @@ __global__ __launch_bounds__(256) void k_gather(ParticleArgs a) {
         continue;
       }
     }
+    T rel[3] = {T(0), T(0), T(0)};
+    const T B = porosity_at<T, D>(P, x, eps, rel);
     bool own_box, own_solid;
     if constexpr (LOCAL) {
       lo.test(a, p, x, !fplbm && B < T(1.0), eps, own_box, own_solid);
@@ -681,6 +670,8 @@ __global__ __launch_bounds__(256) void k_gather(ParticleArgs a) {
       continue;
     }
     if (B >= T(1.0)) continue;
+    T fi[Q], fo[Q];
+    gather_pops<L, S, T>(a, x, fi, fo);
     T mom[3] = {T(0.0), T(0.0), T(0.0)};
 #pragma unroll
     for (int i = 1; i < Q; ++i) {
