@@ -638,17 +638,19 @@ lbm_status lbm_ctx_create(lbm_ctx** out, int32_t lattice, int32_t storage,
   // threads; 128 cells where blocks of 256 would leave over a third of their
   // lanes without a cell (rows of 257 to 341 cells; us per step at 300 x 100 x 60:
   // D3Q19 F32 73 for 84, F64 115 for 149, F16 40 for 46, D3Q27 F32 103 for 118;
-  // at 400 and 520 cells 256 are as fast or faster).  D3Q27 FP64 has one or two
-  // wavefronts per SIMD, and takes one-row blocks of 64 or 128 cells, whichever
-  // leaves fewer lanes idle, which end sooner: 128 x 100 x 60 52 us for 66, 64^3 21
-  // for 28, 256 x 128 x 64 177 for 181.
+  // at 400 and 520 cells 256 are as fast or faster).  D3Q27 FP64 has two
+  // wavefronts per SIMD.  Rows beyond 64 cells take one-row blocks of 64 or 128 of
+  // them, whichever leaves fewer lanes idle, which end sooner: 128 x 100 x 60 52 us for
+  // 66, 256 x 128 x 64 177 for 181.  Shorter rows stay stacked, as one-row blocks are
+  // single wavefronts, too many to start for a small lattice: 33 x 30 x 24 6.4 us
+  // stacked, 8.4 not; 64^3 21 both ways.
   int bx = 64;
   while (bx < 256 && uint64_t(bx) < n[0]) bx *= 2;
   auto lanes = [&](uint64_t w) { return (n[0] + w - 1) / w * w; };
   if (bx == 256 && (lanes(256) - n[0]) * 3 > lanes(256) && n[0] > 256) bx = 128;
   c->shape.bx = bx;
   c->shape.by = 256 / bx;
-  if (lattice == LBM_D3Q27 && storage == LBM_F64) {
+  if (lattice == LBM_D3Q27 && storage == LBM_F64 && n[0] > 64) {
     c->shape.bx = lanes(64) < lanes(128) ? 64 : 128;
     c->shape.by = 1;
   }
