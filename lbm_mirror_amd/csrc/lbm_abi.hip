@@ -134,7 +134,8 @@ struct lbm_ctx {
   uint32_t* owner = nullptr;
   // scatter porosity kept by the gathers' sweeps (ParticleArgs::boxes):
   // kBoxInts ints per particle; por_fresh once the porosity is 1 outside the
-  // previous boxes (after a full reset, kept by every sweep since)
+  // previous boxes (after a full reset, kept by every sweep since) and in the
+  // cells whose operator stamps its own
   int32_t* boxes = nullptr;
   bool por_fresh = false;
   double bin = 1.0;
@@ -275,6 +276,7 @@ bool sweep_eligible(const lbm_ctx* c) {
   return c->np > 0 && c->boxes && c->pp.coupling != LBM_COUPLING_FPLBM &&
          c->pp.porosity_mode == LBM_POROSITY_SCATTER && !c->owner;
 }
+bool stamps_disc(const OpDev& o) { return o.coll == LBM_COLL_PSM && (o.flags & LBM_OPF_PSM_STAMP_DISC); }
 bool sweep_ready(const lbm_ctx* c) { return sweep_eligible(c) && c->por_fresh; }
 
 // Before the couplings of a call: one full reset (porosity 1, no previous
@@ -693,6 +695,8 @@ lbm_status lbm_set_flags(lbm_ctx* c, const uint8_t* flags) {
   HIP_TRY(hipMemcpyAsync(c->flags, flags, c->N, hipMemcpyHostToDevice, c->stream));
   HIP_TRY(hipStreamSynchronize(c->stream));
   c->flags_set = true;
+  for (const OpDev& o : c->ops_h)  // cells may have lost the operator that stamped them
+    if (stamps_disc(o)) c->por_fresh = false;
   return LBM_OK;
 }
 
@@ -780,6 +784,7 @@ lbm_status lbm_set_operator(lbm_ctx* c, uint8_t flag, const lbm_op_desc* op) {
     lbm_status s = ensure_field(c, &c->force, size_t(c->D) * c->N, 0.0);
     if (s) return s;
   }
+  if (stamps_disc(c->ops_h[flag])) c->por_fresh = false;
   c->ops_h[flag] = o;
   c->has_op[flag] = true;
   HIP_TRY(hipSetDevice(c->device));

@@ -1,0 +1,69 @@
+"""The kept porosity (no per-cell reset while particles move) where something
+other than a gather has changed what a reset would give: an operator that
+stamps a fixed disc into the porosity and is then replaced, and cells that get
+another flag.  The oracle resets every cell before each coupling.  Heavy discs:
+the fluid's force, whose sums differ in order, moves none."""
+import numpy as np
+import pytest
+
+from helpers import channel_flags_2d, make_particle
+from lbm_mirror_amd import abi
+
+pytestmark = pytest.mark.gpu
+
+EXT = (96, 60)
+KINDS = [(abi.COUPLING_PSM, abi.COLL_PSM), (abi.COUPLING_HLBM, abi.COLL_HLBM)]
+
+
+def _sims(orc, make, coupling, coll):
+    rng = np.random.default_rng(3)
+    N = EXT[0] * EXT[1]
+    flags = channel_flags_2d(*EXT).reshape(EXT[1], EXT[0])
+    flags[20:40, 60:80] = 5
+    _, Q, _, w, _ = orc.lattice(abi.D2Q9)
+    f0 = np.outer(w, np.ones(N)) * (1 + 0.01 * rng.uniform(-1, 1, size=(Q, N)))
+    stamp = abi.op_desc(collision=abi.COLL_PSM, tau=0.8, flags=abi.OPF_PSM_STAMP_DISC, disc=(70.0, 30.0, 0.0, 6.0, 1.5))
+    part = make_particle([30.0, 30.0], 5.0, 1.5, 2, abi.F64, vel=[0.03, 0.02], mass=1e12, inertia=1e12)
+    prm = abi.particle_params(k_n=0.0, zeta_n=0.0, sub_steps=1, eps=1.5, max_radius=5.0, walls=False, coupling=coupling)
+    out = []
+    for mk in make:
+        s = mk()
+        s.set_flags(flags.reshape(-1))
+        s.set_periodic(1)
+        s.set_operator(1, abi.op_desc(boundary=abi.BC_BOUNCE_BACK))
+        for fl in (2, 3, 4):
+            s.set_operator(fl, abi.op_desc(collision=coll, tau=0.8))
+        s.set_operator(5, stamp)
+        s.set_populations(f0)
+        s.particles_set([part], prm)
+        out.append(s)
+    return flags, out
+
+
+def _both(orc, coupling, coll):
+    from lbm_mirror_amd.lattice import Lattice
+    flags, (g, o) = _sims(orc, [lambda: Lattice(abi.D2Q9, abi.F64, EXT), lambda: orc.Sim(abi.D2Q9, abi.F64, EXT)],
+                          coupling, coll)
+    o.match_gpu_arithmetic()
+    return flags, g, o
+
+
+@pytest.mark.parametrize("what", ["operator", "flags"])
+@pytest.mark.parametrize("coupling,coll", KINDS)
+def test_a_stamped_disc_goes_with_its_operator(hip, orc, coupling, coll, what):
+    flags, g, o = _both(orc, coupling, coll)
+    for s in (g, o):
+        s.step(4)
+    assert np.array_equal(g.get_porosity(), o.get_porosity())
+    assert g.get_porosity().reshape(EXT[1], EXT[0])[30, 70] == 0.0
+    for s in (g, o):
+        if what == "operator":
+            s.set_operator(5, abi.op_desc(collision=coll, tau=0.8))
+        else:
+            s.set_flags(np.where(flags == 5, 2, flags).astype(np.uint8).reshape(-1))
+    for n in (1, 40):
+        for s in (g, o):
+            s.step(n)
+        assert np.array_equal(g.get_porosity(), o.get_porosity())
+        assert np.allclose(g.get_populations(), o.get_populations(), rtol=0, atol=1e-12)
+    g.close()
