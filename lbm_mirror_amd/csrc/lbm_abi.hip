@@ -993,7 +993,7 @@ lbm_status lbm_step(lbm_ctx* c, uint64_t t0, uint64_t nsteps) {
   HIP_TRY(hipSetDevice(c->device));
   const MultiPlan multi = multi_of(c);
   HIP_TRY(hipEventRecord(c->ev0, c->stream));
-  s = prepare_sweep(c);  // (outside any step graph)
+  if (nsteps > 0) s = prepare_sweep(c);  // (outside any step graph)
   if (s) return s;
   // FPLBM reads the stored macro velocity of non-fluid cells every step
   const bool every = c->np > 0 && c->pp.coupling == LBM_COUPLING_FPLBM;

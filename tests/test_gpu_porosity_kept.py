@@ -1,8 +1,9 @@
 """The kept porosity (no per-cell reset while particles move) where something
 other than a gather has changed what a reset would give: an operator that
-stamps a fixed disc into the porosity and is then replaced, and cells that get
-another flag.  The oracle resets every cell before each coupling.  Heavy discs:
-the fluid's force, whose sums differ in order, moves none."""
+stamps a fixed disc into the porosity and is then replaced, cells that get
+another flag, and calls of no steps, which change nothing.  The oracle resets
+every cell before each coupling.  Heavy discs: the fluid's force, whose sums
+differ in order, moves none."""
 import numpy as np
 import pytest
 
@@ -66,4 +67,18 @@ def test_a_stamped_disc_goes_with_its_operator(hip, orc, coupling, coll, what):
             s.step(n)
         assert np.array_equal(g.get_porosity(), o.get_porosity())
         assert np.allclose(g.get_populations(), o.get_populations(), rtol=0, atol=1e-12)
+    g.close()
+
+
+@pytest.mark.parametrize("coupling,coll", KINDS)
+def test_no_steps_change_nothing(hip, orc, coupling, coll):
+    _, g, _ = _both(orc, coupling, coll)
+    g.step(3)
+    por = np.random.default_rng(1).uniform(0, 1, EXT[0] * EXT[1])
+    g.set_porosity(por)
+    sums = g.get_hlbm_sums() if coupling == abi.COUPLING_HLBM else ()
+    g.step(0)
+    assert np.array_equal(g.get_porosity(), por)
+    for a, b in zip(sums, g.get_hlbm_sums()):
+        assert np.array_equal(a, b)
     g.close()
