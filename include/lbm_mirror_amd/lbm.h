@@ -305,9 +305,10 @@ lbm_status lbm_last_step_ms(lbm_ctx* ctx, double* ms);
  * keeps the fastest shape; `chosen->us` is the chosen shape's time per phase.
  * Call it from an even step count, after flags and operators are set.
  * D2Q9 lattices without particles run most steps several per launch, with a
- * second population buffer where the GPU has memory to spare; the tuned shape
- * then runs the others.  After lbm_set_step_tuning every step is a launch of
- * its own in the shape that was set. */
+ * second population buffer where the GPU has memory to spare (freed when a
+ * later call of this library runs out of memory; every step is then a launch
+ * of its own); the tuned shape runs the others.  After lbm_set_step_tuning
+ * every step is a launch of its own in the shape that was set. */
 typedef struct lbm_step_tuning {
   int32_t block_x;  /* threads per block along x: 64, 128 or 256     */
   int32_t form[2];  /* per AA phase (even, odd): 0 default, 1 global, 2 buffer, 3 pairs */

@@ -13,6 +13,7 @@
 #include <cstdio>
 
 #include "../../include/lbm_mirror_amd/lbm.h"
+#include "memory.hpp"
 
 lbm_status lbmx_report(lbm_status s, const char* msg);
 
@@ -86,10 +87,10 @@ extern "C" lbm_status lbm_hbm_ceiling(int32_t device, int32_t kind, uint64_t byt
   CEIL_TRY(hipStreamCreateWithFlags(&s, hipStreamNonBlocking), "hipStreamCreate");
   CEIL_TRY(hipEventCreate(&e0), "hipEventCreate");
   CEIL_TRY(hipEventCreate(&e1), "hipEventCreate");
-  CEIL_TRY(hipMalloc(&a, used), "hipMalloc");
+  CEIL_TRY(lbmx::device_alloc(&a, used), "hipMalloc");
   CEIL_TRY(hipMemsetAsync(a, 0, used, s), "hipMemsetAsync");
   if (kind == LBM_CEILING_COPY) {
-    CEIL_TRY(hipMalloc(&b, used), "hipMalloc");
+    CEIL_TRY(lbmx::device_alloc(&b, used), "hipMalloc");
     CEIL_TRY(hipMemsetAsync(b, 0, used, s), "hipMemsetAsync");
   }
   const unsigned grid = unsigned((n + 255) / 256);

@@ -18,6 +18,7 @@
 
 #include "fields.hpp"
 #include "kernels.hpp"
+#include "memory.hpp"
 #include "readback.hpp"
 
 using namespace lbmx;
@@ -151,9 +152,8 @@ struct lbm_ctx {
   double* res_partial = nullptr;
   double* res_out = nullptr;
   // multi-step launches (D2Q9): the buffer they write to before they come back
-  // to f, asked for once; one_step while a launch shape was set by hand
-  void* f2 = nullptr;
-  bool f2_asked = false;
+  // to f; one_step while a launch shape was set by hand
+  Spare f2;
   bool one_step = false;
   size_t tsz() const { return compute_double(storage) ? 8 : 4; }
   size_t fbytes() const { return size_t(Q) * Np * storage_bytes(storage); }
@@ -162,7 +162,7 @@ struct lbm_ctx {
 namespace {
 
 hipError_t alloc_zero(void** p, size_t bytes, hipStream_t s) {
-  hipError_t e = hipMalloc(p, bytes);
+  hipError_t e = device_alloc(p, bytes);
   if (e != hipSuccess) return e;
   return hipMemsetAsync(*p, 0, bytes, s);
 }
@@ -174,7 +174,7 @@ lbm_status ensure_field(lbm_ctx* c, void** field, size_t count, double fill) {
   if (fill != 0.0) {
     std::vector<double> h(count, fill);
     double* tmp = nullptr;
-    HIP_TRY(hipMalloc(&tmp, count * sizeof(double)));
+    HIP_TRY(device_alloc(&tmp, count * sizeof(double)));
     HIP_TRY(hipMemcpyAsync(tmp, h.data(), count * sizeof(double), hipMemcpyHostToDevice, c->stream));
     HIP_TRY(field_from_double(compute_double(c->storage), *field, tmp, count, c->stream));
     HIP_TRY(hipStreamSynchronize(c->stream));
@@ -209,7 +209,7 @@ Geometry geom(const lbm_ctx* c) {
 lbm_status put_field(lbm_ctx* c, void* field, const double* host, size_t count, int as = -1) {
   double* tmp = nullptr;
   HIP_TRY(hipSetDevice(c->device));
-  HIP_TRY(hipMalloc(&tmp, count * sizeof(double)));
+  HIP_TRY(device_alloc(&tmp, count * sizeof(double)));
   HIP_TRY(hipMemcpyAsync(tmp, host, count * sizeof(double), hipMemcpyHostToDevice, c->stream));
   HIP_TRY(field_from_double(compute_double(as < 0 ? c->storage : as), field, tmp, count, c->stream));
   HIP_TRY(hipStreamSynchronize(c->stream));
@@ -419,7 +419,6 @@ StepArgs step_args(const lbm_ctx* c, uint64_t t, bool write_macros, const uint64
   a.t_dev = t_dev;
   a.write_macros = write_macros ? 1 : 0;
   a.status = c->status_d;
-  a.f2 = c->f2;
   classify(c, a);
   return a;
 }
@@ -435,29 +434,13 @@ bool multi_operators(const lbm_ctx* c) {
   return true;
 }
 
-// A spare buffer of `bytes`, or null where it would leave less than a quarter
-// of the GPU's memory free: the one-step kernels need none.
-void* spare_buffer(size_t bytes) {
-  size_t free_b = 0, total = 0;
-  void* p = nullptr;
-  if (hipMemGetInfo(&free_b, &total) != hipSuccess || free_b < bytes || free_b - bytes < total / 4 ||
-      hipMalloc(&p, bytes) != hipSuccess) {
-    (void)hipGetLastError();
-    return nullptr;
-  }
-  return p;
-}
-
-// The shapes of this lattice's multi-step launches (n = 0: it has none).
-MultiPlan multi_of(lbm_ctx* c) {
+// The shapes of this lattice's multi-step launches, which need its spare buffer
+// (n = 0: it has none, or its steps go one by one).
+bool multi_wanted(const lbm_ctx* c) { return !c->one_step && c->np == 0 && c->n[1] < 65536 && multi_operators(c); }
+MultiPlan multi_of(const lbm_ctx* c, const void* f2) {
   MultiPlan plan;
   std::memset(&plan, 0, sizeof plan);
-  if (c->one_step || c->np > 0 || !multi_operators(c)) return plan;
-  if (!c->f2_asked) {
-    c->f2_asked = true;
-    c->f2 = spare_buffer(c->fbytes());
-  }
-  if (c->f2 && c->n[1] < 65536) plan = multi_plan(c->storage, c->N);
+  if (f2 && multi_wanted(c)) plan = multi_plan(c->storage, c->N);
   return plan;
 }
 
@@ -468,12 +451,12 @@ const MultiShape* multi_fit(const MultiPlan& plan, uint64_t steps) {
   return nullptr;
 }
 
-// 2 * sh.steps steps from phase 0: into the spare buffer and back
-lbm_status multi_pass(lbm_ctx* c, const MultiShape& sh, uint64_t t, const uint64_t* t_dev = nullptr) {
+// 2 * sh.steps steps from phase 0: into the spare buffer f2 and back
+lbm_status multi_pass(lbm_ctx* c, const MultiShape& sh, void* f2, uint64_t t, const uint64_t* t_dev = nullptr) {
   StepArgs a = step_args(c, t, false, t_dev);
-  HIP_TRY(launch_multi(c->storage, sh, a, c->f, c->f2, c->stream));
+  HIP_TRY(launch_multi(c->storage, sh, a, c->f, f2, c->stream));
   a.t = t + uint64_t(sh.steps);
-  HIP_TRY(launch_multi(c->storage, sh, a, c->f2, c->f, c->stream));
+  HIP_TRY(launch_multi(c->storage, sh, a, f2, c->f, c->stream));
   return LBM_OK;
 }
 
@@ -516,13 +499,13 @@ void append_bytes(std::vector<uint8_t>& k, const X& x) {
 // *t_dev by its length, so one graph serves every start step, inside the
 // ramps or past them; *t_dev is set only where a replay does not continue
 // the previous one.
-lbm_status replay_steps(lbm_ctx* c, uint64_t t, bool every, const MultiPlan& multi) {
-  if (!c->t_dev) HIP_TRY(hipMalloc((void**)&c->t_dev, sizeof(uint64_t)));
+lbm_status replay_steps(lbm_ctx* c, uint64_t t, bool every, const MultiPlan& multi, void* f2) {
   std::vector<uint8_t> key;
   append_bytes(key, step_args(c, 0, every, c->t_dev));
   append_bytes(key, c->shape);
   append_bytes(key, c->steps_per_graph);
   append_bytes(key, multi);
+  append_bytes(key, f2);
   append_bytes(key, c->np);
   if (c->np > 0) {
     ParticleArgs pa = particle_args(c);
@@ -541,7 +524,7 @@ lbm_status replay_steps(lbm_ctx* c, uint64_t t, bool every, const MultiPlan& mul
     for (uint32_t i = 0; i < c->steps_per_graph && !s;) {
       const MultiShape* sh = c->phase == 0 ? multi_fit(multi, c->steps_per_graph - i) : nullptr;
       if (sh) {
-        s = multi_pass(c, *sh, i, c->t_dev);
+        s = multi_pass(c, *sh, f2, i, c->t_dev);
         i += 2u * uint32_t(sh->steps);
         continue;
       }
@@ -668,9 +651,10 @@ lbm_status lbm_ctx_destroy(lbm_ctx* c) {
   if (!c) return LBM_OK;
   (void)hipSetDevice(c->device);
   if (c->stream) (void)hipStreamSynchronize(c->stream);
+  c->f2.give_back();
   void* ptrs[] = {c->f, c->flags, c->ops, c->rho, c->u, c->force, c->por, c->bcvel, c->pn, c->pd,
                   c->parts, c->snap, c->f64, c->t64, c->partial, c->cl_count, c->cl_slot,
-                  c->cl_overflow, c->owner, c->t_dev, c->u_prev, c->res_partial, c->res_out, c->boxes, c->f2};
+                  c->cl_overflow, c->owner, c->t_dev, c->u_prev, c->res_partial, c->res_out, c->boxes};
   for (void* p : ptrs)
     if (p) (void)hipFree(p);
   if (c->status_h) (void)hipHostFree(c->status_h);
@@ -790,6 +774,7 @@ lbm_status lbm_set_operator(lbm_ctx* c, uint8_t flag, const lbm_op_desc* op) {
   HIP_TRY(hipSetDevice(c->device));
   HIP_TRY(hipMemcpyAsync(c->ops + flag, &o, sizeof(OpDev), hipMemcpyHostToDevice, c->stream));
   HIP_TRY(hipStreamSynchronize(c->stream));
+  if (!multi_operators(c)) c->f2.give_back();
   return LBM_OK;
 }
 
@@ -860,7 +845,7 @@ lbm_status lbm_set_populations_layout(lbm_ctx* c, const double* f, int32_t layou
   const size_t cnt = population_count(c->lattice, geom(c), layout);
   double* tmp = nullptr;
   HIP_TRY(hipSetDevice(c->device));
-  HIP_TRY(hipMalloc(&tmp, cnt * sizeof(double)));
+  HIP_TRY(device_alloc(&tmp, cnt * sizeof(double)));
   HIP_TRY(hipMemcpyAsync(tmp, f, cnt * sizeof(double), hipMemcpyHostToDevice, c->stream));
   HIP_TRY(pack_populations(c->lattice, c->storage, c->f, tmp, geom(c), c->stream, layout));
   HIP_TRY(hipStreamSynchronize(c->stream));
@@ -876,7 +861,7 @@ lbm_status lbm_get_populations_layout(lbm_ctx* c, double* f, int32_t layout) {
   const size_t cnt = population_count(c->lattice, geom(c), layout);
   double* tmp = nullptr;
   HIP_TRY(hipSetDevice(c->device));
-  HIP_TRY(hipMalloc(&tmp, cnt * sizeof(double)));
+  HIP_TRY(device_alloc(&tmp, cnt * sizeof(double)));
   if (layout == LBM_LAYOUT_REF_AOS_GHOST)  // the ghost ring holds zeros
     HIP_TRY(hipMemsetAsync(tmp, 0, cnt * sizeof(double), c->stream));
   HIP_TRY(unpack_populations(c->lattice, c->storage, c->f, tmp, geom(c), c->phase, c->stream, layout));
@@ -991,7 +976,10 @@ lbm_status lbm_step(lbm_ctx* c, uint64_t t0, uint64_t nsteps) {
   s = report_faults(c);  // of earlier calls' work that has run
   if (s) return s;
   HIP_TRY(hipSetDevice(c->device));
-  const MultiPlan multi = multi_of(c);
+  if (c->steps_per_graph > 0 && !c->t_dev) HIP_TRY(device_alloc(&c->t_dev, sizeof(uint64_t)));
+  if (nsteps > 0 && multi_wanted(c)) c->f2.ask(c->fbytes(), c->stream);
+  const SpareHold spare(c->f2);  // (behind this call's allocations)
+  const MultiPlan multi = multi_of(c, spare.p);
   HIP_TRY(hipEventRecord(c->ev0, c->stream));
   if (nsteps > 0) s = prepare_sweep(c);  // (outside any step graph)
   if (s) return s;
@@ -1009,7 +997,7 @@ lbm_status lbm_step(lbm_ctx* c, uint64_t t0, uint64_t nsteps) {
     // a whole graph of steps: from phase 0, and never the last step of the
     // call (it writes the macros), nor the one before it when tracking
     if (G > 0 && c->phase == 0 && nsteps - k > G + (track ? 1u : 0u)) {
-      s = replay_steps(c, t, every, multi);
+      s = replay_steps(c, t, every, multi, spare.p);
       if (s) return s;
       k += G;
       continue;
@@ -1017,7 +1005,7 @@ lbm_status lbm_step(lbm_ctx* c, uint64_t t0, uint64_t nsteps) {
     const uint64_t silent = nsteps - k - 1;  // steps before the one that writes the macros
     const MultiShape* sh = c->phase == 0 ? multi_fit(multi, track && silent > 0 ? silent - 1 : silent) : nullptr;
     if (sh) {
-      s = multi_pass(c, *sh, t);
+      s = multi_pass(c, *sh, spare.p, t);
       if (s) return s;
       k += 2u * uint64_t(sh->steps);
       continue;
@@ -1122,6 +1110,8 @@ lbm_status lbm_set_step_tuning(lbm_ctx* c, const lbm_step_tuning* t) {
   c->shape.form[0] = t->form[0];
   c->shape.form[1] = t->form[1];
   c->one_step = true;  // every step in this shape
+  HIP_TRY(hipSetDevice(c->device));
+  c->f2.give_back();
   return LBM_OK;
 }
 
@@ -1153,7 +1143,7 @@ lbm_status lbm_autotune(lbm_ctx* c, uint32_t rounds, lbm_step_tuning* chosen) {
   for (const auto& fl : fields) {
     if (!fl.first) continue;
     Saved v{fl.first, nullptr, fl.second};
-    hipError_t e = hipMalloc(&v.copy, v.bytes);
+    hipError_t e = device_alloc(&v.copy, v.bytes);
     if (e == hipSuccess) e = hipMemcpyAsync(v.copy, v.field, v.bytes, hipMemcpyDeviceToDevice, c->stream);
     saved.push_back(v);
     if (e != hipSuccess) {
@@ -1319,6 +1309,7 @@ lbm_status lbm_particles_set(lbm_ctx* c, const lbm_particle* p, uint32_t n,
   HIP_TRY(hipStreamSynchronize(c->stream));
   const int st = particle_storage(c->storage, *prm);
   const bool dbl = compute_double(st);
+  if (n > 0) c->f2.give_back();
   // (re)allocate
   if (n != c->np || dbl != c->pdbl) {
     void* ptrs[] = {c->parts, c->snap, c->f64, c->t64, c->partial, c->boxes};
@@ -1531,8 +1522,7 @@ struct lbm_batch {
   size_t mtiles_cap = 0;
   MultiPlan multi{};
   uint32_t mbegin[4] = {};  // the tiles of multi.shape[i]: [mbegin[i], mbegin[i + 1])
-  void* spare = nullptr;
-  bool spare_asked = false;
+  Spare spare;
   bool one_step = false;
   hipGraphExec_t chain = nullptr;
   uint64_t chain_len = 0;
@@ -1596,12 +1586,10 @@ lbm_status build_tiles(lbm_batch* b) {
     at[m] = bytes;
     bytes += (b->members[m]->fbytes() + 255) / 256 * 256;
   }
-  if (ok && !b->spare_asked) {
-    b->spare_asked = true;
-    b->spare = spare_buffer(bytes);
-  }
-  ok = ok && b->spare;
-  b->multi = ok ? multi_plan(b->storage, cells) : MultiPlan{};
+  b->spare.let_go();  // (for this call's allocations)
+  if (ok) b->spare.ask(bytes, b->stream);
+  else if (!b->one_step) b->spare.give_back();
+  b->multi = ok && b->spare.taken() ? multi_plan(b->storage, cells) : MultiPlan{};
   std::vector<Tile> mtiles;
   for (int i = 0; i < b->multi.n; ++i) {
     const MultiShape& sh = b->multi.shape[i];
@@ -1620,7 +1608,6 @@ lbm_status build_tiles(lbm_batch* b) {
   }
   for (uint32_t m = 0; m < M; ++m) {
     lbm_ctx* c = b->members[m];
-    args[m] = member_args(c, ok ? static_cast<char*>(b->spare) + at[m] : nullptr);
     begin[m] = uint32_t(tiles.size());
     if (!b->active[m]) continue;
     const uint64_t per = uint64_t(bx) * uint64_t(rows);
@@ -1630,19 +1617,25 @@ lbm_status build_tiles(lbm_batch* b) {
   HIP_TRY(hipStreamSynchronize(b->stream));
   if (tiles.size() > b->tiles_cap) {
     if (b->d_tiles) HIP_TRY(hipFree(b->d_tiles));
+    b->d_tiles = nullptr;
     if (b->d_partial) HIP_TRY(hipFree(b->d_partial));
-    b->tiles_cap = std::max<size_t>(tiles.size(), 1);
-    HIP_TRY(hipMalloc((void**)&b->d_tiles, b->tiles_cap * sizeof(Tile)));
-    HIP_TRY(hipMalloc((void**)&b->d_partial, b->tiles_cap * 2 * sizeof(double)));
+    b->d_partial = nullptr;
+    b->tiles_cap = 0;
+    HIP_TRY(device_alloc(&b->d_tiles, tiles.size() * sizeof(Tile)));
+    HIP_TRY(device_alloc(&b->d_partial, tiles.size() * 2 * sizeof(double)));
+    b->tiles_cap = tiles.size();
   }
   b->ntiles = uint32_t(tiles.size());
   if (mtiles.size() > b->mtiles_cap) {
     if (b->d_mtiles) HIP_TRY(hipFree(b->d_mtiles));
     b->d_mtiles = nullptr;
     b->mtiles_cap = 0;
-    HIP_TRY(hipMalloc((void**)&b->d_mtiles, mtiles.size() * sizeof(Tile)));
+    HIP_TRY(device_alloc(&b->d_mtiles, mtiles.size() * sizeof(Tile)));
     b->mtiles_cap = mtiles.size();
   }
+  char* f2 = static_cast<char*>(b->spare.hold());
+  if (!f2) b->multi.n = 0;
+  for (uint32_t m = 0; m < M; ++m) args[m] = member_args(b->members[m], f2 ? f2 + at[m] : nullptr);
   if (!mtiles.empty())
     HIP_TRY(hipMemcpyAsync(b->d_mtiles, mtiles.data(), mtiles.size() * sizeof(Tile), hipMemcpyHostToDevice, b->stream));
   if (!tiles.empty())
@@ -1734,6 +1727,12 @@ lbm_status run_chain(lbm_batch* b, uint64_t t0, uint64_t n, bool with_res, hipEv
   return LBM_OK;
 }
 
+// The spare buffer, held since the tiles were built, until the end of a call.
+struct BatchCall {
+  lbm_batch* b;
+  ~BatchCall() { b->spare.let_go(); }
+};
+
 lbm_status batch_ready(lbm_batch* b) {
   for (lbm_ctx* c : b->members) {
     lbm_status s = check_ready(c);
@@ -1777,11 +1776,11 @@ lbm_status lbm_batch_create(lbm_batch** out, int32_t lattice, int32_t storage, u
   if (hipStreamCreateWithFlags(&b->stream, hipStreamNonBlocking) != hipSuccess ||
       hipEventCreate(&b->ev0) != hipSuccess || hipEventCreate(&b->ev1) != hipSuccess)
     return bail(fail(LBM_ERR_CRITICAL, "stream/event creation"));
-  hipError_t e = hipMalloc((void**)&b->d_members, count * sizeof(StepArgs));
-  if (e == hipSuccess) e = hipMalloc((void**)&b->d_tile_begin, (count + 1) * sizeof(uint32_t));
-  if (e == hipSuccess) e = hipMalloc((void**)&b->d_uprev, count * sizeof(void*));
-  if (e == hipSuccess) e = hipMalloc((void**)&b->d_res, 2 * count * sizeof(double));
-  if (e == hipSuccess) e = hipMalloc((void**)&b->d_t0, sizeof(uint64_t));
+  hipError_t e = device_alloc(&b->d_members, count * sizeof(StepArgs));
+  if (e == hipSuccess) e = device_alloc(&b->d_tile_begin, (count + 1) * sizeof(uint32_t));
+  if (e == hipSuccess) e = device_alloc(&b->d_uprev, count * sizeof(void*));
+  if (e == hipSuccess) e = device_alloc(&b->d_res, 2 * count * sizeof(double));
+  if (e == hipSuccess) e = device_alloc(&b->d_t0, sizeof(uint64_t));
   if (e == hipSuccess)
     e = hipMemcpy(b->d_uprev, b->uprev.data(), count * sizeof(void*), hipMemcpyHostToDevice);
   if (e != hipSuccess) return bail(fail(LBM_ERR_OUT_OF_MEMORY, "batch arrays: %s", hipGetErrorString(e)));
@@ -1794,10 +1793,11 @@ lbm_status lbm_batch_destroy(lbm_batch* b) {
   (void)hipSetDevice(b->device);
   if (b->stream) (void)hipStreamSynchronize(b->stream);
   drop_chain(b);
+  b->spare.give_back();
   for (void* p : b->uprev) (void)hipFree(p);
   for (lbm_ctx* c : b->members) lbm_ctx_destroy(c);
   void* ptrs[] = {b->d_members, b->d_tiles, b->d_tile_begin, b->d_uprev, b->d_partial,
-                  b->d_res,     b->d_t0,    b->d_mtiles,     b->spare};
+                  b->d_res,     b->d_t0,    b->d_mtiles};
   for (void* p : ptrs)
     if (p) (void)hipFree(p);
   if (b->ev0) (void)hipEventDestroy(b->ev0);
@@ -1821,6 +1821,7 @@ lbm_status lbm_batch_step(lbm_batch* b, uint64_t t0, uint64_t nsteps) {
   lbm_status s = batch_ready(b);
   if (s) return s;
   HIP_TRY(hipSetDevice(b->device));
+  const BatchCall call{b};
   if (b->tiles_dirty) {
     s = build_tiles(b);
     if (s) return s;
@@ -1848,6 +1849,7 @@ lbm_status lbm_batch_run(lbm_batch* b, uint64_t t0, double tol, uint64_t check_e
   lbm_status s = batch_ready(b);
   if (s) return s;
   HIP_TRY(hipSetDevice(b->device));
+  const BatchCall call{b};
   const uint32_t M = uint32_t(b->members.size());
   std::vector<uint64_t> steps(M, 0);
   std::vector<double> res(M, 0.0), sums(2 * M);
@@ -1859,6 +1861,9 @@ lbm_status lbm_batch_run(lbm_batch* b, uint64_t t0, double tol, uint64_t check_e
     uint64_t cells = 0;
     for (uint32_t m = 0; m < M; ++m)
       if (b->active[m]) cells += b->members[m]->N;
+    // an allocation that waits for the spare buffer has it between two chains
+    b->spare.let_go();
+    if (!b->spare.hold() && b->multi.n > 0) b->tiles_dirty = true;
     s = run_chain(b, t0 + done, n, true, b->ev0);
     if (s) return s;
     HIP_TRY(hipEventRecord(b->ev1, b->stream));
@@ -1906,6 +1911,8 @@ lbm_status lbm_batch_set_tuning(lbm_batch* b, const lbm_batch_tuning* t) {
   b->shape.grid = t->grid;
   b->one_step = true;  // every step in this shape
   b->tiles_dirty = true;
+  HIP_TRY(hipSetDevice(b->device));
+  b->spare.give_back();
   return LBM_OK;
 }
 
@@ -1936,7 +1943,7 @@ lbm_status lbm_batch_autotune(lbm_batch* b, lbm_batch_tuning* chosen) {
     void* srcs[3] = {c->f, c->u, c->rho};
     for (int k = 0; k < 3; ++k) {
       void* p = nullptr;
-      HIP_TRY(hipMalloc(&p, sizes[k]));
+      HIP_TRY(device_alloc(&p, sizes[k]));
       HIP_TRY(hipMemcpyAsync(p, srcs[k], sizes[k], hipMemcpyDeviceToDevice, b->stream));
       saved.push_back(p);
     }
@@ -1952,6 +1959,7 @@ lbm_status lbm_batch_autotune(lbm_batch* b, lbm_batch_tuning* chosen) {
     bool &flag, was;
     ~Pin() { flag = was; }
   } pin{b->one_step, b->one_step};
+  const BatchCall call{b};
   b->one_step = true;
   const int blocks[3] = {64, 128, 256}, rows_c[3] = {1, 2, 4}, grids[4] = {0, 4, 8, 16};
   for (int bi = 0; bi < 3; ++bi)

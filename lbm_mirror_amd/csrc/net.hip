@@ -27,6 +27,7 @@
 #include <vector>
 
 #include "../../include/lbm_mirror_amd/lbm.h"
+#include "memory.hpp"
 #include "readback.hpp"
 
 namespace lbmnet {
@@ -1101,7 +1102,7 @@ template <class T>
 lbm_status dalloc(T** p, size_t count) {
   *p = nullptr;
   if (count == 0) return LBM_OK;
-  NET_TRY(hipMalloc(reinterpret_cast<void**>(p), count * sizeof(T)));
+  NET_TRY(lbmx::device_alloc(p, count * sizeof(T)));
   // done when this returns: the network's stream does not wait for the null
   // stream's work, and a copy queued there could be cleared after it
   NET_TRY(hipMemset(*p, 0, count * sizeof(T)));
