@@ -11,6 +11,7 @@
 
 #include <algorithm>
 #include <condition_variable>
+#include <cstdlib>
 #include <mutex>
 #include <thread>
 #include <vector>
@@ -33,6 +34,7 @@ struct Stage {
   int device = 0;
   char* mem = nullptr;
   size_t size = 0;
+  bool pinned = true;
   hipEvent_t ev[kSlots] = {};
 };
 
@@ -43,7 +45,8 @@ std::vector<Stage>* g_free = nullptr;  // (never destroyed: no HIP call after ma
 void drop(Stage& t) {
   for (hipEvent_t e : t.ev)
     if (e) (void)hipEventDestroy(e);
-  if (t.mem) (void)hipHostFree(t.mem);
+  if (t.mem && t.pinned) (void)hipHostFree(t.mem);
+  else std::free(t.mem);
   t = Stage();
 }
 
@@ -70,6 +73,12 @@ hipError_t take(int device, size_t size, Stage& t) {
   t.device = device;
   t.size = size;
   hipError_t e = hipHostMalloc((void**)&t.mem, size, hipHostMallocDefault);
+  if (e != hipSuccess) {  // no pinned memory: ordinary memory, through the runtime's own staging
+    (void)hipGetLastError();
+    t.pinned = false;
+    t.mem = static_cast<char*>(std::malloc(size));
+    e = t.mem ? hipSuccess : hipErrorOutOfMemory;
+  }
   for (int i = 0; i < kSlots && e == hipSuccess; ++i) e = hipEventCreateWithFlags(&t.ev[i], hipEventDisableTiming);
   if (e != hipSuccess) drop(t);
   return e;
@@ -78,7 +87,7 @@ hipError_t take(int device, size_t size, Stage& t) {
 void give(Stage& t) {
   {
     std::lock_guard<std::mutex> lock(g_mu);
-    if (g_users > 0) {
+    if (g_users > 0 && t.pinned) {
       if (!g_free) {
         g_free = new std::vector<Stage>();
         g_free->reserve(kKept);

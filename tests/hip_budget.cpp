@@ -1,5 +1,6 @@
 // A GPU of little memory: hipMalloc, hipFree and hipMemGetInfo of whatever is
-// loaded after this library, within a budget of bytes.
+// loaded after this library, within a budget of bytes; and a host whose pinned
+// memory is used up (hipHostMalloc).
 #include <dlfcn.h>
 #include <hip/hip_runtime_api.h>
 
@@ -10,6 +11,7 @@ namespace {
 std::mutex mu;
 std::map<void*, size_t> blocks;
 size_t budget = 0, used = 0;
+bool pinned = true;
 template <class F>
 F real(const char* name) {
   return reinterpret_cast<F>(dlsym(RTLD_NEXT, name));
@@ -19,6 +21,7 @@ F real(const char* name) {
 extern "C" {
 void budget_set(size_t bytes) { budget = bytes; }
 size_t budget_used() { return used; }
+void pinned_set(int left) { pinned = left != 0; }
 
 hipError_t hipMalloc(void** p, size_t bytes) {
   static const auto f = real<hipError_t (*)(void**, size_t)>("hipMalloc");
@@ -46,5 +49,9 @@ hipError_t hipMemGetInfo(size_t* free_b, size_t* total) {
   *free_b = budget - used;
   *total = budget;
   return hipSuccess;
+}
+hipError_t hipHostMalloc(void** p, size_t bytes, unsigned flags) {
+  static const auto f = real<hipError_t (*)(void**, size_t, unsigned)>("hipHostMalloc");
+  return pinned ? f(p, bytes, flags) : hipErrorOutOfMemory;
 }
 }
