@@ -40,7 +40,8 @@ struct Stage {
 
 std::mutex g_mu;
 int g_users = 0;
-std::vector<Stage>* g_free = nullptr;  // (never destroyed: no HIP call after main)
+Stage g_free[kKept];  // (never destroyed: no HIP call after main)
+size_t g_kept = 0;
 
 void drop(Stage& t) {
   for (hipEvent_t e : t.ev)
@@ -54,19 +55,17 @@ hipError_t take(int device, size_t size, Stage& t) {
   Stage small;  // one that is in the way
   {
     std::lock_guard<std::mutex> lock(g_mu);
-    if (g_free) {
-      for (size_t i = 0; i < g_free->size(); ++i) {
-        Stage& f = (*g_free)[i];
-        if (f.device != device || f.size < size) continue;
-        t = f;
-        g_free->erase(g_free->begin() + i);
-        return hipSuccess;
-      }
-      if (g_free->size() >= kKept) {
-        small = g_free->front();
-        g_free->erase(g_free->begin());
-      }
+    auto pick = [](size_t i) {  // (the others stay in order)
+      const Stage f = g_free[i];
+      for (--g_kept; i < g_kept; ++i) g_free[i] = g_free[i + 1];
+      return f;
+    };
+    for (size_t i = 0; i < g_kept; ++i) {
+      if (g_free[i].device != device || g_free[i].size < size) continue;
+      t = pick(i);
+      return hipSuccess;
     }
+    if (g_kept == kKept) small = pick(0);
   }
   drop(small);
   t = Stage();
@@ -87,15 +86,9 @@ hipError_t take(int device, size_t size, Stage& t) {
 void give(Stage& t) {
   {
     std::lock_guard<std::mutex> lock(g_mu);
-    if (g_users > 0 && t.pinned) {
-      if (!g_free) {
-        g_free = new std::vector<Stage>();
-        g_free->reserve(kKept);
-      }
-      if (g_free->size() < kKept) {
-        g_free->push_back(t);
-        return;
-      }
+    if (g_users > 0 && t.pinned && g_kept < kKept) {
+      g_free[g_kept++] = t;
+      return;
     }
   }
   drop(t);
@@ -178,11 +171,12 @@ hipError_t read_chunks(hipStream_t s, Stage& t, size_t slot, const std::vector<C
 }  // namespace
 
 void read_back_user(int change) {
-  std::vector<Stage> gone;
+  Stage gone[kKept];
   {
     std::lock_guard<std::mutex> lock(g_mu);
     g_users += change;
-    if (g_users == 0 && g_free) gone.swap(*g_free);
+    if (g_users == 0)
+      for (; g_kept > 0; --g_kept) gone[g_kept - 1] = g_free[g_kept - 1];
   }
   for (Stage& t : gone) drop(t);
 }

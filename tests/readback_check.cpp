@@ -1,11 +1,12 @@
 // Read-back (csrc/readback.hip) over a stand-in for the HIP calls it makes:
 // every byte exactly once and in place, whole units, with and without pinned
-// memory, a failing copy, and nothing kept once the last user has gone.
+// memory or heap, a failing copy, and nothing kept once the last user has gone.
 #include <atomic>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
 #include <mutex>
+#include <new>
 #include <set>
 #include <vector>
 
@@ -16,6 +17,7 @@ std::mutex mu;
 std::set<void*> pinned;
 std::atomic<int> events{0}, copies{0};
 bool no_pinned = false;
+bool no_heap = false;
 int fail_copy = -1;
 hipError_t last = hipSuccess;
 
@@ -28,12 +30,23 @@ void check(bool ok, const char* what) {
 #define CHECK(x) check(x, #x)
 }  // namespace
 
+void* operator new(size_t n) {
+  void* p = no_heap ? nullptr : std::malloc(n);
+  if (!p) throw std::bad_alloc();
+  return p;
+}
+void operator delete(void* p) noexcept { std::free(p); }
+void operator delete(void* p, size_t) noexcept { std::free(p); }
+
 extern "C" {
 hipError_t hipHostMalloc(void** p, size_t bytes, unsigned) {
   if (no_pinned) return last = hipErrorOutOfMemory;
   std::lock_guard<std::mutex> lock(mu);
+  const bool was = no_heap;
+  no_heap = false;
   *p = std::malloc(bytes);
   pinned.insert(*p);
+  no_heap = was;
   return hipSuccess;
 }
 hipError_t hipHostFree(void* p) {
@@ -95,6 +108,17 @@ static hipError_t run(const std::vector<size_t>& units, bool whole) {
 
 int main() {
   lbmx::read_back_user(1);
+  {  // where the heap is used up: small reads need none, larger ones say so
+    std::vector<unsigned char> from(12 << 20, 3), to(12 << 20);
+    unsigned char* out = to.data();
+    ReadBack r{from.data(), 1000, 1, [out](const char* data, size_t at, size_t n) { std::memcpy(out + at, data, n); }};
+    no_heap = true;
+    const hipError_t small = lbmx::read_back(0, nullptr, &r, 1);
+    r.bytes = from.size();
+    const hipError_t large = lbmx::read_back(0, nullptr, &r, 1);
+    no_heap = false;
+    CHECK(small == hipSuccess && to[999] == 3 && large == hipErrorOutOfMemory);
+  }
   for (bool none : {false, true}) {
     no_pinned = none;
     for (size_t n : {size_t(1), size_t(1000), size_t(699050), size_t(699051), size_t(2000003)}) {
