@@ -1047,7 +1047,6 @@ double rho_unit(double u_max) { return 3.0 * u_max * u_max; }
 struct Layer {
   int cin, cr, cpad;  // input channels, output channels (real / padded to 8)
   size_t w_off, b_off;
-  size_t p_off = 0;  // of its partial weight-gradient tiles
   uint16_t *wb = nullptr, *wt = nullptr;
   int relu;
   int level;
@@ -1072,7 +1071,15 @@ struct lbm_net {
   float *y = nullptr, *t = nullptr;
   uint8_t* msk = nullptr;
   uint32_t* ftab = nullptr;  // upload_features' words
+  // partial weight-gradient tiles: of all layers, or of as many at a time as the
+  // memory there was holds; those that are not yet added up (reduce_gradients)
   float* partial = nullptr;
+  size_t partial_n = 0, partial_used = 0;
+  struct {
+    int layer, splits;
+    size_t at;
+  } pending[12];
+  int npending = 0;
   double* lpartial = nullptr;
   double* dloss = nullptr;
   float* dlosses = nullptr;
@@ -1097,6 +1104,12 @@ int W_(const lbm_net* n, int l) { return n->cfg.width >> l; }
 int H_(const lbm_net* n, int l) { return n->cfg.height >> l; }
 
 size_t level_pixels(const lbm_net* n, int l) { return size_t(n->cfg.batch) * H_(n, l) * W_(n, l); }
+
+#define NS(expr)                  \
+  do {                            \
+    lbm_status s_ = (expr);       \
+    if (s_ != LBM_OK) return s_;  \
+  } while (0)
 
 template <class T>
 lbm_status dalloc(T** p, size_t count) {
@@ -1160,6 +1173,7 @@ int wgrad_most_splits(const Layer& L, int M) {  // no fewer pixels have more
   const int tiles = ((9 * L.cin + 8 + BM - 1) / BM) * ((L.cpad + bn - 1) / bn);
   return std::max(1, std::min(kWgradBlocks / std::max(1, tiles), (M + 255) / 256));
 }
+size_t wgrad_tile(const Layer& L) { return size_t(9 * L.cin + 8) * L.cpad; }  // floats of a split
 void wgrad_shape(const lbm_net* n, const Layer& L, int B, int& splits, int& chunk) {
   const int M = B * H_(n, L.level) * W_(n, L.level);
   splits = wgrad_most_splits(L, M);
@@ -1188,16 +1202,58 @@ lbm_status conv(lbm_net* n, int li, int B, Act in, Act out, float* outf) {
   return LBM_OK;
 }
 
+// The weight and bias gradients of the layers whose partial tiles wait, into n->g.
+lbm_status reduce_gradients(lbm_net* n) {
+  if (n->npending == 0) return LBM_OK;
+  WredArgs a{};
+  unsigned end = 0;
+  for (int k = 0; k < n->npending; ++k) {
+    const auto& p = n->pending[k];
+    const Layer& L = n->layers[p.layer];
+    end += unsigned(((9 * L.cin + 1) * L.cr + 63) / 64);
+    a.layer[k] = WredLayer{n->partial + p.at, n->g + L.w_off, p.splits, 9 * L.cin, L.cpad, L.cr, end};
+  }
+  n->npending = 0;
+  n->partial_used = 0;
+  hipLaunchKernelGGL(k_wreduce, dim3(end), dim3(256), 0, n->stream, a);
+  NET_TRY(hipGetLastError());
+  return LBM_OK;
+}
+
+// Memory for the partial tiles: of every layer (256 x 256, batch 16, widths 32 to
+// 160: 331 MB), so that one launch adds them all up; where there is not that much,
+// of the largest layer (47 MB).  Every element that is read is written first.
+lbm_status need_partial(lbm_net* n) {
+  if (n->partial) return LBM_OK;
+  size_t all = 0, most = 0;
+  for (const Layer& L : n->layers) {
+    const size_t k = size_t(wgrad_most_splits(L, int(level_pixels(n, L.level)))) * wgrad_tile(L);
+    all += k;
+    most = std::max(most, k);
+  }
+  n->partial_n = all;
+  if (hipMalloc(reinterpret_cast<void**>(&n->partial), all * sizeof(float)) == hipSuccess) return LBM_OK;
+  (void)hipGetLastError();
+  n->partial = nullptr;
+  n->partial_n = most;
+  NET_TRY(lbmx::device_alloc(&n->partial, most * sizeof(float)));
+  return LBM_OK;
+}
+
 // Backward of layer li given its pre-activation gradient dpre: the partial
-// tiles of its weight and bias gradients (reduce_gradients), and (if dx.p) the input gradient, masked by
-// (in > 0) when mask_in.
+// tiles of its weight and bias gradients, behind those that wait where they
+// fit, and (if dx.p) the input gradient, masked by (in > 0) when mask_in.
 lbm_status conv_bwd(lbm_net* n, int li, int B, Act in, Act dpre, Act dx, bool mask_in) {
   const Layer& L = n->layers[li];
   const int H = H_(n, L.level), W = W_(n, L.level);
   int splits, chunk;
   wgrad_shape(n, L, B, splits, chunk);
-  WgradArgs wa{B, H, W, L.cin, L.cpad, in, dpre, n->partial + L.p_off, chunk};
+  const size_t size = size_t(splits) * wgrad_tile(L);
+  if (n->partial_used + size > n->partial_n) NS(reduce_gradients(n));
+  WgradArgs wa{B, H, W, L.cin, L.cpad, in, dpre, n->partial + n->partial_used, chunk};
   NET_TRY(launch_wgrad(wa, splits, n->stream));
+  n->pending[n->npending++] = {li, splits, n->partial_used};
+  n->partial_used += size;
   if (dx.p) {
     ConvArgs a{};
     a.B = B;
@@ -1249,12 +1305,6 @@ lbm_status up_bwd(lbm_net* n, int level, int B, Act gfine, Act gcoarse, int C) {
   return LBM_OK;
 }
 
-#define NS(expr)                  \
-  do {                            \
-    lbm_status s_ = (expr);       \
-    if (s_ != LBM_OK) return s_;  \
-  } while (0)
-
 lbm_status forward(lbm_net* n, int B) {
   const int* w = n->cfg.widths;
   const int cw[3] = {w[1] + w[0], w[2] + w[1], w[3] + w[2]};  // cat widths: [up | skip]
@@ -1293,23 +1343,10 @@ lbm_status loss_fwd(lbm_net* n, int B, double nf, double* dloss, float* dlossf) 
   return LBM_OK;
 }
 
-// Every layer's weight and bias gradient into n->g.
-lbm_status reduce_gradients(lbm_net* n, int B) {
-  WredArgs a{};
-  unsigned end = 0;
-  for (int k = 0; k < 12; ++k) {
-    const Layer& L = n->layers[k];
-    int splits, chunk;
-    wgrad_shape(n, L, B, splits, chunk);
-    end += unsigned(((9 * L.cin + 1) * L.cr + 63) / 64);
-    a.layer[k] = WredLayer{n->partial + L.p_off, n->g + L.w_off, splits, 9 * L.cin, L.cpad, L.cr, end};
-  }
-  hipLaunchKernelGGL(k_wreduce, dim3(end), dim3(256), 0, n->stream, a);
-  NET_TRY(hipGetLastError());
-  return LBM_OK;
-}
-
 lbm_status backward(lbm_net* n, int B) {
+  NS(need_partial(n));
+  n->npending = 0;  // (of a backward pass that failed)
+  n->partial_used = 0;
   const int* w = n->cfg.widths;
   const int cw[3] = {w[1] + w[0], w[2] + w[1], w[3] + w[2]};
   const Act none{nullptr, 0, 0};
@@ -1331,7 +1368,7 @@ lbm_status backward(lbm_net* n, int B) {
   NS(pool_bwd(n, 0, B, act(n->gpool[1], w[0]), act(n->gcat[0], cw[0], w[1]), act(n->cat[0], cw[0], w[1]), w[0]));
   NS(conv_bwd(n, 1, B, act(n->a[0], w[0]), act(n->gcat[0], cw[0], w[1]), act(n->ga[0], w[0]), true));
   NS(conv_bwd(n, 0, B, act(n->x, 8), act(n->ga[0], w[0]), none, false));
-  return reduce_gradients(n, B);
+  return reduce_gradients(n);
 }
 
 lbm_status refresh_weights(lbm_net* n) {
@@ -1499,12 +1536,7 @@ lbm_status create_impl(lbm_net* n) {
   NS(dalloc(&n->t, level_pixels(n, 0) * 3));
   NS(dalloc(&n->msk, level_pixels(n, 0)));
   NS(dalloc(&n->ftab, feature_words(n->cfg, c.batch)));
-  size_t partial = 0;
-  for (Layer& L : n->layers) {
-    L.p_off = partial;
-    partial += size_t(wgrad_most_splits(L, int(level_pixels(n, L.level)))) * (9 * L.cin + 8) * L.cpad;
-  }
-  NS(dalloc(&n->partial, partial));
+  if (c.capacity > 0) NS(need_partial(n));  // (a network that is to be trained)
   NS(dalloc(&n->lpartial, size_t(blocks_for(level_pixels(n, 0)))));
   NS(dalloc(&n->dloss, 1));
   const size_t HW = size_t(c.height) * c.width;
