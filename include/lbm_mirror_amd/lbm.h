@@ -308,7 +308,8 @@ lbm_status lbm_last_step_ms(lbm_ctx* ctx, double* ms);
  * second population buffer where the GPU has memory to spare (freed when a
  * later call of this library runs out of memory; every step is then a launch
  * of its own); the tuned shape runs the others.  After lbm_set_step_tuning
- * every step is a launch of its own in the shape that was set. */
+ * every step is a launch of its own in the shape that was set, whichever it
+ * is, until lbm_autotune chooses one again. */
 typedef struct lbm_step_tuning {
   int32_t block_x;  /* threads per block along x: 64, 128 or 256     */
   int32_t form[2];  /* per AA phase (even, odd): 0 default, 1 global, 2 buffer, 3 pairs */
@@ -443,9 +444,9 @@ lbm_status lbm_batch_run(lbm_batch* b, uint64_t t0, double tol, uint64_t check_e
 /* Times candidate tile shapes on the batch (state restored afterwards) and
  * keeps the fastest. */
 lbm_status lbm_batch_autotune(lbm_batch* b, lbm_batch_tuning* chosen);
-/* After lbm_batch_set_tuning every step is a launch of its own in these tiles
- * (otherwise D2Q9 batches run most steps several per launch, as single
- * lattices do). */
+/* After lbm_batch_set_tuning every step is a launch of its own in these tiles,
+ * until lbm_batch_autotune chooses some again (otherwise D2Q9 batches run most
+ * steps several per launch, as single lattices do). */
 lbm_status lbm_batch_set_tuning(lbm_batch* b, const lbm_batch_tuning* tuning);
 /* Device time and member cell updates of the last step/run call. */
 lbm_status lbm_batch_stats(lbm_batch* b, double* ms, uint64_t* cell_updates);

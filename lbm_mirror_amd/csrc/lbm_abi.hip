@@ -1246,6 +1246,7 @@ lbm_status lbm_autotune(lbm_ctx* c, uint32_t rounds, lbm_step_tuning* chosen) {
   c->shape.by = 1;
   c->shape.form[0] = bf[0];
   c->shape.form[1] = bf[1];
+  c->one_step = false;  // (no longer a shape set by hand)
   if (chosen) {
     chosen->block_x = widths[bw];
     chosen->form[0] = bf[0];
@@ -1953,11 +1954,11 @@ lbm_status lbm_batch_autotune(lbm_batch* b, lbm_batch_tuning* chosen) {
   const BatchShape keep = b->shape;
   BatchShape best = keep;
   double best_ms = 1e30;
-  // the trials time the one-step launches' tiles; the chains keep their
-  // multi-step launches
+  // the trials time the one-step launches' tiles; the chains have their
+  // multi-step launches afterwards, also where a shape had been set by hand
   struct Pin {
-    bool &flag, was;
-    ~Pin() { flag = was; }
+    bool &flag, then;
+    ~Pin() { flag = then; }
   } pin{b->one_step, b->one_step};
   const BatchCall call{b};
   b->one_step = true;
@@ -1990,6 +1991,7 @@ lbm_status lbm_batch_autotune(lbm_batch* b, lbm_batch_tuning* chosen) {
   if (s) return s;
   for (void* p : saved) (void)hipFree(p);
   b->shape = best;
+  pin.then = false;
   b->tiles_dirty = true;
   if (chosen) {
     chosen->block = best.block;
