@@ -116,7 +116,10 @@ def hbm_ceilings(L, device=0):
 def bench_c1(args):
     """Config 1: D2Q9 FP64 channel 256x64, parabolic Zou/He inlet u_max 0.05,
     pressure outlet, tau 0.8, from rest; reports MLUPS and the developed
-    centre-line velocity against the analytic parabola (flux-normalised)."""
+    centre-line velocity against the analytic parabola (flux-normalised).
+    A short run from rest goes before the timed one: the first call of a process
+    loads the kernels' code and captures the step graph inside its timed events
+    (18 ms, 0.9 us on each of 20000 steps)."""
     import numpy as np
     from lbm_mirror_amd import abi
     from lbm_mirror_amd.lattice import Lattice
@@ -129,6 +132,9 @@ def bench_c1(args):
     lat.set_boundary_velocity(parabolic_inlet(nx, ny, 0.05))
     lat.init_equilibrium(1.0, (0.0, 0.0))
     steps = args.steps if args.steps != 1000 else 20000
+    lat.step(100, t0=0)
+    lat.init_equilibrium(1.0, (0.0, 0.0))
+    lat.sync()
     lat.step(steps, t0=0)
     lat.sync()
     ms = lat.last_step_ms()
@@ -145,9 +151,9 @@ def bench_c1(args):
             "vs_baseline": None, "dtype": "f64", "data": "synthetic",
             "config": {"workload": "D2Q9 BGK channel 256x64, Zou/He velocity inlet u_max 0.05, "
                                    "pressure outlet rho 1, BB walls, tau 0.8, from rest"},
-            "roofline": {"bound": "hbm", "achieved": round(nx * ny * 144 / (ms / steps * 1e-3) / 1e9, 1),
-                         "peak": HBM_PEAK_GBS, "unit": "GB/s",
-                         "frac": round(nx * ny * 144 / (ms / steps * 1e-3) / 1e9 / HBM_PEAK_GBS, 4),
+            # several steps per read of the populations: no fraction of the HBM peak
+            "roofline": {"bound": "launch latency", "achieved": round(nx * ny * 144 / (ms / steps * 1e-3) / 1e9, 1),
+                         "peak": None, "unit": "GB/s of a run that reads and writes every step", "frac": None,
                          "traffic": None},
             "analytic": {"fitted_u_max": round(scale, 6),
                          "max_shape_error_rel": round(err, 5)}}
@@ -235,8 +241,9 @@ def bench_c3(args, storage):
 
 def bench_c4(args):
     """Config 4: 256 D2Q9 lattices, sides ~U[64,512], seeded obstacles 5-20%
-    solid (r~U[4,24]), u_max~U[0.01,0.08], tau~U[0.55,1.2]; one launch per
-    step over all members (autotuned tiles), run towards residual 1e-6."""
+    solid (r~U[4,24]), u_max~U[0.01,0.08], tau~U[0.55,1.2]; one launch for
+    several steps over all members (the others in autotuned tiles), run
+    towards residual 1e-6."""
     import numpy as np
     from lbm_mirror_amd import abi
     from lbm_mirror_amd.lattice import Batch
@@ -256,7 +263,7 @@ def bench_c4(args):
     steps, res = b.run(tol=1e-6, check_every=200, max_steps=max_steps)
     ms, upd = b.stats()
     cells = sum(int(np.prod(m[0])) for m in ms_)
-    return {"metric": "aggregate MLUPS (256 ragged D2Q9 lattices, one launch per step)",
+    return {"metric": "aggregate MLUPS (256 ragged D2Q9 lattices, several steps per launch)",
             "value": round(upd / (ms * 1e3), 1), "unit": "MLUPS", "n_gpus": 1,
             "steps": int(steps.max()), "warmup": 0, "ms_per_step": None,
             "higher_is_better": True, "scaling": "weak", "vs_baseline": None, "dtype": "f32",
@@ -264,9 +271,9 @@ def bench_c4(args):
             "config": {"workload": f"{args.members} D2Q9 lattices, sides U[64,512], {cells} cells",
                        "tuning": tune, "converged_1e-6": int(np.sum(res < 1e-6)),
                        "median_steps": float(np.median(steps)), "wall_device_ms": round(ms, 2)},
-            "roofline": {"bound": "hbm", "achieved": round(upd * 72 / (ms * 1e-3) / 1e9, 1),
-                         "peak": HBM_PEAK_GBS, "unit": "GB/s",
-                         "frac": round(upd * 72 / (ms * 1e-3) / 1e9 / HBM_PEAK_GBS, 4), "traffic": None}}
+            # several steps per read of the populations: no fraction of the HBM peak
+            "roofline": {"bound": "valu", "achieved": round(upd * 72 / (ms * 1e-3) / 1e9, 1), "peak": None,
+                         "unit": "GB/s of a run that reads and writes every step", "frac": None, "traffic": None}}
 
 
 def _c5_batch(members, warm=None, storage=None):
