@@ -28,6 +28,7 @@
 
 #include "../../include/lbm_mirror_amd/lbm.h"
 #include "memory.hpp"
+#include "net_init.hpp"
 #include "readback.hpp"
 
 namespace lbmnet {
@@ -1547,11 +1548,12 @@ lbm_status create_impl(lbm_net* n) {
   }
   // He-normal initialisation, biases zero
   std::vector<float> hw(n->nparam, 0.f);
-  std::mt19937_64 rng(c.seed);
-  for (const Layer& L : n->layers) {
-    std::normal_distribution<double> nd(0.0, std::sqrt(2.0 / (9.0 * L.cin)));
-    for (size_t i = 0; i < size_t(9) * L.cin * L.cr; ++i) hw[L.w_off + i] = float(nd(rng));
+  HeLayer he[12];
+  for (int k = 0; k < 12; ++k) {
+    const Layer& L = n->layers[k];
+    he[k] = {hw.data() + L.w_off, size_t(9) * L.cin * L.cr, L.cin};
   }
+  he_normal(c.seed, he, 12);
   NET_TRY(hipMemcpy(n->w, hw.data(), n->nparam * sizeof(float), hipMemcpyHostToDevice));
   NS(refresh_weights(n));
   NET_TRY(hipStreamSynchronize(n->stream));
