@@ -444,6 +444,12 @@ MultiPlan multi_of(const lbm_ctx* c, const void* f2) {
   return plan;
 }
 
+// Whether a call or chain of n steps, whose last one writes the macros, has room
+// for the plan's shortest pair of launches (if not it needs no spare buffer).
+bool multi_room(const MultiPlan& plan, uint64_t n) {
+  return plan.n > 0 && n > 2u * uint64_t(plan.shape[plan.n - 1].steps);
+}
+
 // The longest pair of launches of the plan within `steps` steps, or null.
 const MultiShape* multi_fit(const MultiPlan& plan, uint64_t steps) {
   for (int i = 0; i < plan.n; ++i)
@@ -977,7 +983,7 @@ lbm_status lbm_step(lbm_ctx* c, uint64_t t0, uint64_t nsteps) {
   if (s) return s;
   HIP_TRY(hipSetDevice(c->device));
   if (c->steps_per_graph > 0 && !c->t_dev) HIP_TRY(device_alloc(&c->t_dev, sizeof(uint64_t)));
-  if (nsteps > 0 && multi_wanted(c)) c->f2.ask(c->fbytes(), c->stream);
+  if (multi_wanted(c) && multi_room(multi_plan(c->storage, c->N), nsteps)) c->f2.ask(c->fbytes(), c->stream);
   const SpareHold spare(c->f2);  // (behind this call's allocations)
   const MultiPlan multi = multi_of(c, spare.p);
   HIP_TRY(hipEventRecord(c->ev0, c->stream));
@@ -1515,6 +1521,7 @@ struct lbm_batch {
   uint32_t ntiles = 0;
   size_t tiles_cap = 0;
   bool tiles_dirty = true;
+  uint64_t tiles_for = 0;  // the longest chain that the tiles were built for
   // captured chains: key = (length, with residual)
   // multi-step launches: their work list (active members' tiles) and one spare
   // buffer for every member's populations; one_step while a tile shape was
@@ -1569,7 +1576,8 @@ void drop_chain(lbm_batch* b) {
 }
 
 // Tiles of the active members, member by member; members' argument records.
-lbm_status build_tiles(lbm_batch* b) {
+// For chains of up to n steps: short ones need no tiles of multi-step launches.
+lbm_status build_tiles(lbm_batch* b, uint64_t n) {
   const uint32_t M = uint32_t(b->members.size());
   std::vector<StepArgs> args(M);
   std::vector<Tile> tiles;
@@ -1577,20 +1585,22 @@ lbm_status build_tiles(lbm_batch* b) {
   const int bx = b->shape.block, rows = b->shape.rows;
   HIP_TRY(hipSetDevice(b->device));
   // multi-step launches where every member's operators allow them
-  bool ok = !b->one_step;
+  bool able = true;
   uint64_t cells = 0;
   size_t bytes = 0;
   std::vector<size_t> at(M, 0);
   for (uint32_t m = 0; m < M; ++m) {
-    ok = ok && multi_operators(b->members[m]);
+    able = able && multi_operators(b->members[m]);
     if (b->active[m]) cells += b->members[m]->N;
     at[m] = bytes;
     bytes += (b->members[m]->fbytes() + 255) / 256 * 256;
   }
   b->spare.let_go();  // (for this call's allocations)
+  if (!able) b->spare.give_back();
+  b->multi = multi_plan(b->storage, cells);
+  const bool ok = able && !b->one_step && multi_room(b->multi, n);
   if (ok) b->spare.ask(bytes, b->stream);
-  else if (!b->one_step) b->spare.give_back();
-  b->multi = ok && b->spare.taken() ? multi_plan(b->storage, cells) : MultiPlan{};
+  if (!ok || !b->spare.taken()) b->multi = MultiPlan{};
   std::vector<Tile> mtiles;
   for (int i = 0; i < b->multi.n; ++i) {
     const MultiShape& sh = b->multi.shape[i];
@@ -1645,6 +1655,7 @@ lbm_status build_tiles(lbm_batch* b) {
   HIP_TRY(hipMemcpyAsync(b->d_tile_begin, begin.data(), (M + 1) * sizeof(uint32_t), hipMemcpyHostToDevice, b->stream));
   HIP_TRY(hipStreamSynchronize(b->stream));
   b->tiles_dirty = false;
+  b->tiles_for = n;
   drop_chain(b);
   return LBM_OK;
 }
@@ -1697,8 +1708,8 @@ lbm_status enqueue_chain(lbm_batch* b, uint64_t n, bool with_res) {
 // `start` (if given) is recorded after any capture, right before the chain's
 // work, so a timed region never holds the host's capture and instantiation.
 lbm_status run_chain(lbm_batch* b, uint64_t t0, uint64_t n, bool with_res, hipEvent_t start = nullptr) {
-  if (b->tiles_dirty) {
-    lbm_status s = build_tiles(b);
+  if (b->tiles_dirty || n > b->tiles_for) {
+    lbm_status s = build_tiles(b, n);
     if (s) return s;
   }
   const bool graphable = (n % 2 == 0) && b->phase == 0;
@@ -1823,10 +1834,8 @@ lbm_status lbm_batch_step(lbm_batch* b, uint64_t t0, uint64_t nsteps) {
   if (s) return s;
   HIP_TRY(hipSetDevice(b->device));
   const BatchCall call{b};
-  if (b->tiles_dirty) {
-    s = build_tiles(b);
-    if (s) return s;
-  }
+  s = build_tiles(b, nsteps);
+  if (s) return s;
   s = run_chain(b, t0, nsteps, false, b->ev0);
   if (s) return s;
   HIP_TRY(hipEventRecord(b->ev1, b->stream));
@@ -1970,7 +1979,7 @@ lbm_status lbm_batch_autotune(lbm_batch* b, lbm_batch_tuning* chosen) {
         b->shape.rows = rows_c[ri];
         b->shape.grid = grids[gi] == 0 ? 0 : grids[gi] * cus;
         b->tiles_dirty = true;
-        s = build_tiles(b);
+        s = build_tiles(b, 8);
         if (s) return s;
         // warm-up with the timed chain's length: the timed call then replays
         // the graph this one captured (no capture inside the timed region)

@@ -1,7 +1,7 @@
 """The second population buffer of D2Q9 lattices and batches is spare: it goes
 when another lattice, batch or network needs the GPU's memory, and when no
-step can use it any more.  The lattices then run on, step by step, with the
-same results.  Each case runs in a process of its own, on a GPU that
+step can use it any more; a call of too few steps for it does not take it.  The
+lattices then run on, step by step, with the same results.  Each case runs in a process of its own, on a GPU that
 hip_budget.cpp makes small."""
 import ctypes as C
 import os
@@ -11,7 +11,8 @@ import sys
 import pytest
 
 HERE = os.path.dirname(os.path.abspath(__file__))
-CASES = ["lattice_lattice", "lattice_network", "batch_batch", "shape", "operator", "particles", "tiles"]
+CASES = ["lattice_lattice", "lattice_network", "batch_batch", "shape", "operator", "particles", "tiles",
+         "short", "shortbatch"]
 EXT = (1024, 500)
 SPARE = 9 * 4 * EXT[0] * EXT[1]  # FP32
 MB = 1 << 20
@@ -67,6 +68,17 @@ def _main(so, case):
         return b
 
     has, _, needs = case.partition("_")
+    if case.startswith("short"):
+        a = lattice() if case == "short" else batch()
+        before = used()
+        for n in (1, 2, 4, 3):
+            a.step(n)
+            assert used() - before < SPARE // 2
+        a.step(5)
+        assert used() - before >= SPARE
+        a.step(1)
+        a.close()
+        return
     if not needs:
         a = batch() if case == "tiles" else lattice()
         before = used()
