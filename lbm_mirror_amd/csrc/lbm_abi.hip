@@ -1522,7 +1522,6 @@ struct lbm_batch {
   size_t tiles_cap = 0;
   bool tiles_dirty = true;
   uint64_t tiles_for = 0;  // the longest chain that the tiles were built for
-  // captured chains: key = (length, with residual)
   // multi-step launches: their work list (active members' tiles) and one spare
   // buffer for every member's populations; one_step while a tile shape was
   // set by hand or is being timed
@@ -1532,6 +1531,7 @@ struct lbm_batch {
   uint32_t mbegin[4] = {};  // the tiles of multi.shape[i]: [mbegin[i], mbegin[i + 1])
   Spare spare;
   bool one_step = false;
+  // captured chains: key = (length, with residual)
   hipGraphExec_t chain = nullptr;
   uint64_t chain_len = 0;
   int chain_res = -1;

@@ -22,11 +22,16 @@
 // its neighbours write), so launches come in pairs that end in the first
 // buffer, in the natural layout.
 //
-// Measured against one-step launches, us per step: 256x64 4.19 -> 2.14 (F64),
-// 3.87 -> 1.82 (F32); 512x256 7.2 -> 5.2, 5.4 -> 3.2; 1023x517 15.4 -> 11.2,
-// 11.4 -> 6.8; 2048x2048 111 -> 63, 51.7 -> 32.3 (130 GLUPS; the populations'
-// traffic is then 2.9 TB/s and the instructions bound it), F16 38.5 -> 26.5;
-// 128 uneven lattices with 10.3 M cells 504 -> 171, 162 -> 86.
+// Measured against one-step launches in their tuned shape, us per step in F64,
+// F32, F16, BF16: 256x64 3.67 -> 2.07, 3.56 -> 1.75, 3.17 -> 1.76, 3.19 -> 1.79;
+// 512x256 5.32 -> 4.07, 4.66 -> 3.14, 4.26 -> 3.13, 4.25 -> 3.25; 1023x517 15.0 ->
+// 11.4, 9.97 -> 6.85, 8.24 -> 6.33, 8.29 -> 6.54; 2048x2048 100 -> 56, 52 -> 28, 31.3 ->
+// 24.5, 31.6 -> 25.8; 128 uneven lattices with 10.3 M cells 504 -> 174, 143 -> 84, 97 ->
+// 75, 108 -> 79.  What bounds it, by counters: with many FP32 cells the issue of
+// vector instructions (at four cycles each all of a launch's cycles: 128 lattices);
+// in FP64, whose tile of shape A leaves room for one block per CU, half of that,
+// the rest waits at the block's barriers; at 1023x517 half; at 256x64, 256 blocks of
+// one pass each, a sixth: the chain of steps inside a launch and the launches.
 #include <hip/hip_runtime.h>
 
 #include <type_traits>
@@ -316,7 +321,18 @@ hipError_t launch_storage(int storage, const MultiShape& sh, const StepArgs* a, 
 
 // By the cells that one launch covers: few cells need many small blocks and
 // long launches, many cells little margin.  F64 leaves C sooner (512x256: C
-// 5.22, D 4.14; F32 C 3.24, D 3.63).
+// 5.22, D 4.14; F32 C 3.24, D 3.63).  Both shapes on both sides of each line, us
+// per step in F64 / F32 / F16 / BF16:
+//   24000   150x150 B 3.20/2.23/2.15/2.19, C 2.83/2.18/2.15/2.19;
+//           170x160 B 3.29/2.28/2.16/2.21, C 2.91/2.22/2.19/2.20 (256x64: B, see above)
+//   100000  (F64) 300x300 C 4.40, D 4.22; 330x330 C 4.60, D 4.22
+//   160000  400x380 C -/3.76/3.74/3.94, D -/3.70/3.61/3.70;
+//           430x400 C -/3.92/3.81/3.99, D -/4.20/4.03/4.13
+//   800000  900x850 D 14.5/8.22/7.79/8.13, A 14.3/8.44/7.96/8.37;
+//           950x890 D 14.5/8.69/8.41/8.69, A 14.8/8.70/8.15/8.61
+// At the lines the shapes differ by less than at a factor of two to either side:
+// 13% at most (F64 at 22,500 cells).  A batch counts all its members' cells,
+// whatever their widths.
 MultiPlan multi_plan(int storage, uint64_t cells) {
   const uint64_t long_until = storage == LBM_F64 ? 100000 : 160000;
   if (cells <= 24000) return {3, {kShapes[kShapeB], kShapes[kShapeE], kShapes[kShapeF]}};

@@ -985,7 +985,6 @@ __global__ void k_standardize(float* t, size_t n, float m0, float m1, float m2, 
   t[i] = (t[i] - m) / sd;
 }
 
-// Minibatch assembly from the on-device training set.
 // Network input from the lattices' flags and the words of upload_features: 16
 // bytes a pixel.  (Laid out by the host this was 16 of the 20 ms of 16
 // predictions of 256 x 256.)
@@ -1001,6 +1000,7 @@ __global__ void k_features(const uint8_t* flags, const uint32_t* tab, int B, int
       make_uint4(open | (own << 16), (own >> 16) | (row << 16), (col & 0xffffu) | (row & 0xffff0000u), at);
 }
 
+// Minibatch assembly from the on-device training set.
 __global__ void k_gather(const uint16_t* xs, const float* ts, const uint8_t* ms, const uint32_t* idx, int B, int HW,
                          uint16_t* x, float* t, uint8_t* m) {
   const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;  // (the batch's pixels fit an int)
@@ -1222,8 +1222,8 @@ lbm_status reduce_gradients(lbm_net* n) {
 }
 
 // Memory for the partial tiles: of every layer (256 x 256, batch 16, widths 32 to
-// 160: 331 MB), so that one launch adds them all up; where there is not that much,
-// of the largest layer (47 MB).  Every element that is read is written first.
+// 160: 331 MiB), so that one launch adds them all up; where there is not that much,
+// of the largest layer (47 MiB).  Every element that is read is written first.
 lbm_status need_partial(lbm_net* n) {
   if (n->partial) return LBM_OK;
   size_t all = 0, most = 0;
