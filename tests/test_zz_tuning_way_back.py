@@ -8,7 +8,7 @@ import sys
 
 import pytest
 
-from test_gpu_spare_memory import HERE, small_gpu  # noqa: F401
+from test_zz_spare_memory import HERE, small_gpu  # noqa: F401
 
 
 @pytest.mark.gpu
