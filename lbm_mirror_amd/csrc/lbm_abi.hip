@@ -434,8 +434,8 @@ bool multi_operators(const lbm_ctx* c) {
   return true;
 }
 
-// The shapes of this lattice's multi-step launches, which need its spare buffer
-// (n = 0: it has none, or its steps go one by one).
+// Whether this lattice's steps may share launches, and the shapes of such
+// launches, which need its spare buffer (n = 0: it has none).
 bool multi_wanted(const lbm_ctx* c) { return !c->one_step && c->np == 0 && c->n[1] < 65536 && multi_operators(c); }
 MultiPlan multi_of(const lbm_ctx* c, const void* f2) {
   MultiPlan plan;
